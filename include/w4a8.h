@@ -130,9 +130,11 @@ int w4a8_topk_no_alloc(const float *y, int n, int k, float *vals, int32_t *idx, 
  *     through ggml's vector expf; the input of down (:858-860). y = W Q8_0(a).
  * Each is byte-identical to the standalone producer below followed by
  * w4a8_gemv. x, norm_w and gate_up 16-byte aligned; the fused rmsnorm takes
- * k <= 8192 (its float64 squares are staged in LDS), the standalone one any k.
- * The float64 sum is n / 4 dependent adds whatever the hardware: about 8 ns
- * each here, the latency the reference's summation order costs. */
+ * k <= 8192, the standalone one any k.
+ * The float64 sum is taken in parallel with a bound on the reference order's
+ * result, and in that order itself only where the bound does not settle the
+ * float32 it rounds to.
+ */
 int w4a8_gemv_rmsnorm(const void *w, const float *x, const float *norm_w, float eps, float *y, int rows, int k,
                       void *stream);
 int w4a8_gemv_rmsnorm_argmax(const void *w, const float *x, const float *norm_w, float eps, float *y, int rows, int k,

@@ -148,7 +148,7 @@ int w4a8_topk_no_alloc(const float *y, int n, int k, float *vals, int32_t *idx, 
     return hip_status(launch_topk_no_alloc(y, n, k, vals, idx, (hipStream_t)stream));
 }
 
-// The fused rmsnorm stages x's float64 squares in LDS: k <= 8192.
+// The fused rmsnorm's range of k.
 constexpr int RMS_FUSED_MAX_K = 8192;
 
 int w4a8_gemv_rmsnorm(const void *w, const float *x, const float *norm_w, float eps, float *y, int rows, int k,

@@ -319,7 +319,7 @@ int chain_plan_create(const w4a8_plan_step *steps, int n, bool overlapped, w4a8_
             const int waves = gate_up_silu_waves(s.rows, s.k);
             sh.grid = tiles / 2 / (waves / 2);
             sh.threads = 64 * waves;
-            sh.lds = (size_t)waves * TILE_BYTES + x_lds_bytes(s.k / QK) + (rms ? rms_sq_doubles(s.k) * 8 + 16 : 0);
+            sh.lds = (size_t)waves * TILE_BYTES + x_lds_bytes(s.k / QK);
         }
         PlanArgs a;
         std::memset(&a, 0, sizeof a);

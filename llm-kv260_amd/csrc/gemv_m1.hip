@@ -73,9 +73,8 @@ size_t argmax_workspace_bytes() { return ARGMAX_KEY_OFFSET + 64; }
 
 M1Shape gemv_m1_shape(int tiles, int k, XFormat xf, bool /*argmax*/, int cus) {
     const int nb = k / QK;
-    // Staged activation: int8 values, fp32 scale and int32 sum per block; for
-    // X_RMS also the squares of x as float64 and the rmsnorm scale.
-    const size_t x_lds = x_lds_bytes(nb) + (xf == X_RMS ? rms_sq_doubles(k) * 8 + 16 : 0);
+    // Staged activation: int8 values, fp32 scale and int32 sum per block.
+    const size_t x_lds = x_lds_bytes(nb);
     // Launch shape, from what bounds each size:
     //  * Small matrices (at most two tiles per CU): latency. One tile per
     //    wave, two-wave workgroups spread over the CUs (each stages its own
@@ -220,8 +219,7 @@ hipError_t launch_gemv_gate_up_silu(const uint8_t *w, const float *x, XFormat xf
     const int half = P.tiles / 2;
     const int nb = k / QK;
     const int grid = half / (waves / 2);
-    const size_t x_lds = x_lds_bytes(nb) + (xf == X_RMS ? rms_sq_doubles(k) * 8 + 16 : 0);
-    const size_t lds = (size_t)waves * TILE_BYTES + x_lds;
+    const size_t lds = (size_t)waves * TILE_BYTES + x_lds_bytes(nb);
     if (q8) {
         if (xf == X_RMS) return launch_pass<X_RMS, true, true, false, PAIR_Q8>(P, grid, 64 * waves, lds, stream);
         return launch_pass<X_F32, true, true, false, PAIR_Q8>(P, grid, 64 * waves, lds, stream);

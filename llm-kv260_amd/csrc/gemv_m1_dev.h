@@ -194,9 +194,8 @@ __device__ __forceinline__ void load_tile(const GemvParams &P, int tile, int lan
 }
 
 // LDS layout (dynamic): per-wave slabs [waves][9216] | the staged activation
-// (nb / 8 columns of XCOL_DWORDS) | for X_RMS the float64 squares of x
-// (rms_sq_doubles(k), chain by chain) and the scale. `block` / `nblocks` are this workgroup's index and the
-// number of workgroups sharing the matrix.
+// (nb / 8 columns of XCOL_DWORDS). `block` / `nblocks` are this workgroup's
+// index and the number of workgroups sharing the matrix.
 // ONE_PASS: a tile holds at most eight rows (K >= 2048), so one pass of the
 // ordered sums covers it and each lane stores at most one value per tile.
 // The workgroup's best key (its waves' keys through LDS) goes into the
@@ -397,52 +396,38 @@ __device__ __forceinline__ void gemv_m1_body(const GemvParams &P, int block, int
     auto stage_x = [&]() {
         float rms = 0.0f;
         if constexpr (XF == X_RMS) {
-            // rmsnorm's scale needs the whole of x: its squares go to LDS as
-            // float64 after the staged x (chain by chain, rms_sq_index), wave
-            // 0 reduces them, and the scale comes back through LDS. Block b's
-            // elements 32 b + 4 m + c are square 8 b + m of chain c.
-            double *sq = reinterpret_cast<double *>(s_x + (nb / 8) * XCOL_DWORDS);
-            float *s_rms = reinterpret_cast<float *>(sq + rms_sq_doubles(P.k));
-            const int cs = P.k / 4 + 2;
-            auto squares = [&](const XRaw<XF> &r, int b) {
-                double *c0 = sq + 8 * b;
-#pragma unroll
-                for (int m = 0; m < 8; ++m) {
-                    const double a = r.v[m].x, c = r.v[m].y, d = r.v[m].z, e = r.v[m].w;
-                    c0[m] = a * a;
-                    c0[cs + m] = c * c;
-                    c0[2 * cs + m] = d * d;
-                    c0[3 * cs + m] = e * e;
-                }
+            // rmsnorm's scale needs the whole of x: each thread's squares,
+            // then one sum over the workgroup (rms_scale_block, its partials
+            // in wave 0's slab, which no tile has reached yet).
+            double p = 0.0;
+            auto square = [&](const float4 &v) {
+                const double a = v.x, b = v.y, c = v.z, d = v.w;
+                p = fma(a, a, p);
+                p = fma(b, b, p);
+                p = fma(c, c, p);
+                p = fma(d, d, p);
             };
             if (quarter) {
-                // Element 32 b + 4 q + c is square 8 b + q of chain c; element
-                // 32 b + 16 + 4 q + c square 8 b + 4 + q.
                 if (tid < 4 * nb) {
-                    double *c0 = sq + 8 * (tid >> 2) + (tid & 3);
-                    const double a[4] = {xq.xa.x, xq.xa.y, xq.xa.z, xq.xa.w};
-                    const double e[4] = {xq.xb.x, xq.xb.y, xq.xb.z, xq.xb.w};
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        c0[c * cs] = a[c] * a[c];
-                        c0[c * cs + 4] = e[c] * e[c];
-                    }
+                    square(xq.xa);
+                    square(xq.xb);
                 }
             } else {
-                if (tid < nb) squares(xr, tid);
+                auto squares = [&](const XRaw<XF> &r) {
+#pragma unroll
+                    for (int m = 0; m < 8; ++m) square(r.v[m]);
+                };
+                if (tid < nb) squares(xr);
                 for (int b = tid + nthreads; b < nb; b += nthreads) {
                     XRaw<XF> xb;
                     x_load<XF, XAUX>(P.x, P.k, b, true, xb, P.norm_w);
-                    squares(xb, b);
+                    squares(xb);
                 }
             }
-            __syncthreads();
-            if (wave == 0) {
-                const float sc = rms_scale_wave(sq, P.k, P.eps);
-                if (lane == 0) *s_rms = sc;
-            }
-            __syncthreads();
-            rms = *s_rms;
+            const __amdgpu_buffer_rsrc_t xs_rsrc = buffer_of(P.x, (uint32_t)(4 * P.k));
+            rms = rms_scale_block(p, P.k, P.eps, waves, reinterpret_cast<double *>(lds), [&](int i) {
+                return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, 4 * i, 0, XAUX));
+            });
         }
         if (quarter) {
             if constexpr (XF == X_RMS) {

@@ -206,29 +206,18 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
     return sg * u;
 }
 
-// rmsnorm's scale (tp_llama.cpp:557-569) from the float64 squares of x
-// (exact: a float32 square fits a float64), n % 128 == 0: the sum of squares
-// accumulates in float64 in four chains, element i in chain i % 4 in
-// increasing i (the reference's fused multiply-add of an exact square is this
-// add); the chains meet as (c0 + c2) + (c1 + c3); then
-// 1 / sqrtf((float)(ss / n) + eps).
+// rmsnorm's scale (tp_llama.cpp:557-569): the sum of squares accumulates in
+// float64 in four chains, element i in chain i % 4 in increasing i (the
+// reference's fused multiply-add of an exact square is an add of it); the
+// chains meet as (c0 + c2) + (c1 + c3); then 1 / sqrtf((float)(ss / n) + eps).
 //
-// Layout: chain c's squares lie contiguously, square i at rms_sq_index(i, n),
-// each chain n / 4 + 2 doubles after the last; rms_sq_doubles(n) doubles in
-// all, 16-byte aligned. The squares are written by the whole workgroup
-// beforehand, so the chains carry the adds and nothing else.
-//
-// One wave runs the four chains, chain c in row c (lanes 16c .. 16c + 15):
-// lane 16c + i holds chain c's squares 16g + i, g = 0, 1, ..., one 8-byte LDS
-// read per lane per sixteen steps, four reads ahead. Each step is one
-// v_fmac_f64 whose first operand comes through DPP row_newbcast:i (lane i of
-// the row, to every lane of it): acc = sq * 1.0 + acc, the chain's add
-// exactly (the product is exact, the fma rounds once). So a step costs one
-// dependent float64 instruction (about 5.4 clocks at n = 2048: 2,764 for 512
-// steps, where a chain lane reading its own squares from LDS took 4,900-6,300).
-// The whole wave must be active. The result is returned in every lane.
-__host__ __device__ constexpr size_t rms_sq_doubles(int n) { return (size_t)n + 8; }
-__device__ __forceinline__ int rms_sq_index(int i, int n) { return (i & 3) * (n / 4 + 2) + (i >> 2); }
+// The chains are n / 4 dependent float64 adds (1.2 us at n = 2048), but ss is
+// only ever seen through the rounding of ss / n to float32, 29 bits coarser.
+// So the workgroup sums the squares in parallel in any order, bounds how far
+// the chains' sum can lie from that (rms_scale_block), and takes the float32
+// both ends of the interval round to. Where they round apart (about once in
+// 2^18 rows at n = 2048, or a NaN in x) one wave runs the chains as written.
+// The fused decode step of 33 norms: 315.8 us with the chains in each, 275.3 so.
 
 // Sixteen steps of the lane's chain from one read (lane i of the row holds
 // step i). The leading s_nop keeps the DPP source clear of a VALU write in
@@ -259,44 +248,87 @@ __device__ __forceinline__ double rms_row_steps(double acc, double sq, double on
     return acc;
 }
 
-template <int N>
-__device__ __forceinline__ double rms_chain(const double *sq, int n, int lane) {
+// ss / n by the chains, in one whole wave; x_at(i) is element i. Chain c runs
+// in row c of the wave (lanes 16c .. 16c + 15): lane 16c + i squares the
+// chain's elements 16g + i, g = 0, 1, ..., a few reads ahead, and each step is
+// one v_fmac_f64 whose first operand comes through DPP row_newbcast:i (lane i
+// of the row, to every lane of it): acc = sq * 1.0 + acc, the chain's add
+// exactly (the product is exact, the fma rounds once).
+template <class X>
+__device__ __forceinline__ double rms_mean_chains(X x_at, int n) {
     constexpr int AHEAD = 4;                   // reads in flight
-    const int len = N ? N : n;
-    const int groups = len / 64;               // sixteen steps each
-    const double *src = sq + (lane >> 4) * (len / 4 + 2) + (lane & 15);
+    const int lane = threadIdx.x & 63;
+    const int groups = n / 64;                 // sixteen steps each; n % 256 == 0
+    const int first = 4 * (lane & 15) + (lane >> 4);
     const double one = 1.0;
     double acc = 0.0;
-    double buf[AHEAD];
+    for (int g = 0; g < groups; g += AHEAD) {
+        float v[AHEAD];
 #pragma unroll
-    for (int t = 0; t < AHEAD; ++t) buf[t] = t < groups ? src[16 * t] : 0.0;
-    auto round = [&](int g) {
+        for (int t = 0; t < AHEAD; ++t) v[t] = x_at(64 * (g + t) + first);
 #pragma unroll
         for (int t = 0; t < AHEAD; ++t) {
-            if (g + t < groups) {
-                const double v = buf[t];
-                if (g + t + AHEAD < groups) buf[t] = src[16 * (g + t + AHEAD)];
-                acc = rms_row_steps(acc, v, one);
-            }
+            const double a = v[t];
+            acc = rms_row_steps(acc, a * a, one);
         }
-    };
-    if constexpr (N != 0) {
-#pragma unroll
-        for (int g = 0; g < N / 64; g += AHEAD) round(g);
-    } else {
-        for (int g = 0; g < groups; g += AHEAD) round(g);
     }
-    return acc;
+    const double l0 = __shfl(acc, 0), l1 = __shfl(acc, 16), l2 = __shfl(acc, 32), l3 = __shfl(acc, 48);
+    return ((l0 + l2) + (l1 + l3)) / (double)n;
 }
 
-__device__ __forceinline__ float rms_scale_wave(const double *sq, int n, float eps) {
-    const int lane = threadIdx.x & 63;
-    // The hidden size of the decode shapes with its trip count known (the
-    // compiler then unrolls the chain); any other n in a loop.
-    const double acc = n == 2048 ? rms_chain<2048>(sq, n, lane) : rms_chain<0>(sq, n, lane);
-    const double l0 = __shfl(acc, 0), l1 = __shfl(acc, 16), l2 = __shfl(acc, 32), l3 = __shfl(acc, 48);
-    const double ss = (l0 + l2) + (l1 + l3);
-    return 1.0f / sqrtf((float)(ss / (double)n) + eps);
+// The sum over each row of sixteen lanes, the same bits in all of them.
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov_f64(double v) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+__device__ __forceinline__ double row_sum_f64(double v) {
+    v = v + dpp_mov_f64<0xB1>(v);     // quad_perm(1,0,3,2)
+    v = v + dpp_mov_f64<0x4E>(v);     // quad_perm(2,3,0,1)
+    v = v + dpp_mov_f64<0x141>(v);    // row_half_mirror
+    return v + dpp_mov_f64<0x140>(v); // row_mirror
+}
+
+// rmsnorm's scale, in every thread of the workgroup: p is the thread's own sum
+// of squares (float64, any order, at most n / 4 + 16 of them or 0), part
+// 8-byte aligned LDS of RMS_PART(waves) doubles that nothing else uses until
+// the caller's next barrier. Every wave is whole and calls this.
+//
+// The bound. All terms are positive, so a sum that takes at most r rounded
+// adds from any term to the result lies within a factor (1 + 2^-53)^+-r of the
+// exact one: r <= n / 4 + 1 in the chains, r < n / 4 + 48 here (the thread's
+// adds, four row steps, up to four rows of partials, four row steps). The
+// division, 1 / n and the two products below add five roundings more; the
+// slack of e covers them and the second-order terms. Rounding to float32 is
+// monotonic: when both ends of [q (1 - e), q (1 + e)] give one float32, the
+// chains' mean gives it too (an infinity included; a NaN compares unequal).
+__host__ __device__ constexpr int RMS_PART(int waves) { return 4 * waves + 1; }
+
+template <class X>
+__device__ __forceinline__ float rms_scale_block(double p, int n, float eps, int waves, double *part, X x_at) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const double rn = 1.0 / (double)n;
+    const double e = (double)(n / 2 + 128) * 0x1p-53;
+    p = row_sum_f64(p);
+    if ((lane & 15) == 0) part[4 * wave + (lane >> 4)] = p;
+    __syncthreads();
+    double s = 0.0;
+    for (int i = lane & 15; i < 4 * waves; i += 16) s = s + part[i];
+    const double q = row_sum_f64(s) * rn;
+    const float lo = (float)(q * (1.0 - e)), hi = (float)(q * (1.0 + e));
+    float mean = lo;
+    if (!(lo == hi)) {   // the same in every thread: each computed it from the same partials
+        if (wave == 0) {
+            const double m = rms_mean_chains(x_at, n);
+            if (lane == 0) part[4 * waves] = m;
+        }
+        __syncthreads();
+        mean = (float)part[4 * waves];
+    }
+    return 1.0f / sqrtf(mean + eps);
 }
 
 }  // namespace w4a8

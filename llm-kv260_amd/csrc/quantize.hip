@@ -25,47 +25,11 @@ __device__ __forceinline__ void load_block(const float *src, float v[32]) {
     }
 }
 
-// Q8_0 of one 32-element block (q4_0.py:83-97), stored as block b of row `row`
-// of the engine layout (int8[k] | float32[k/32]) or of ggml Q8_0 blocks.
-template <int OUT>
-__device__ __forceinline__ void quantize_store(const float v[32], int row, int b, int k, uint8_t *__restrict__ out) {
-    const int nb = k >> 5;
-    float amax = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 32; ++e) amax = fmaxf(amax, fabsf(v[e]));
-    const float d = q8_scale(amax);
-    const float inv = safe_recip(d);
-    uint32_t q[8];
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
-        uint32_t word = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) word |= ((uint32_t)(uint8_t)q8_round(v[4 * w + e], inv)) << (8 * e);
-        q[w] = word;
-    }
-    const uint16_t dh = float_to_half_bits(d);
-    if constexpr (OUT == X_ENGINE) {
-        uint8_t *rowp = out + (size_t)row * (k + 4 * nb);
-        uint4 *dst = reinterpret_cast<uint4 *>(rowp + 32 * b);
-        dst[0] = make_uint4(q[0], q[1], q[2], q[3]);
-        dst[1] = make_uint4(q[4], q[5], q[6], q[7]);
-        reinterpret_cast<float *>(rowp + k)[b] = half_bits_to_float(dh);
-    } else {
-        uint16_t *dst = reinterpret_cast<uint16_t *>(out + ((size_t)row * nb + b) * Q8_0_BYTES);
-        dst[0] = dh;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            dst[1 + 2 * w] = (uint16_t)(q[w] & 0xFFFFu);
-            dst[2 + 2 * w] = (uint16_t)(q[w] >> 16);
-        }
-    }
-}
-
-// Q8_0 of values 4g .. 4g + 3 of a 32-element block, thread g (0..7) of an
-// aligned group of eight: amax is the group's max (DPP quad_perm [1,0,3,2],
+// Q8_0 (q4_0.py:83-97) of values 4g .. 4g + 3 of a 32-element block, thread g
+// (0..7) of an aligned group of eight, stored in block b of row `row` of the
+// engine layout (int8[k] | float32[k/32]) or of ggml Q8_0 blocks: amax is the group's max (DPP quad_perm [1,0,3,2],
 // [2,3,0,1], then row_half_mirror), so every thread computes the same d and
-// inv as a thread holding the whole block, and its four bytes are the ones
-// quantize_store would write there.
+// inv as a thread holding the whole block.
 template <int OUT>
 __device__ __forceinline__ void quantize_store8(const float4 v, int row, int b, int g, int k, uint8_t *__restrict__ out) {
     const int nb = k >> 5;
@@ -122,40 +86,43 @@ __global__ __launch_bounds__(256) void silu_mul_q8_0_kernel(const float *__restr
 
 // h = rmsnorm(x) * norm_w (tp_llama.cpp:557-569) of m rows of float32[k],
 // quantized to the engine layout: one workgroup per row (the sum of squares
-// runs over the whole row); the squares in LDS as float64 for wave 0's four
-// chains, x read again (from L2) for the normalization.
+// runs over the whole row). Latency: thread t holds the row's float4s t + 256 j
+// (x and the norm weight, all NV of each in flight at once), so x is read once,
+// and eight consecutive threads hold a block, as quantize_store8 takes it.
+template <int NV>
 __global__ __launch_bounds__(256) void rmsnorm_q8_0_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                            float eps, int k, uint8_t *__restrict__ out) {
-    extern __shared__ __attribute__((aligned(16))) double sq[];
-    __shared__ float scale;
-    const int row = blockIdx.x, nb = k >> 5;
+    __shared__ double part[RMS_PART(4)];
+    const int row = blockIdx.x, n4 = k >> 2;
     const float *xr = x + (size_t)row * k;
-    const int cs = k / 4 + 2;     // chain stride (rms_sq_index)
-    for (int i = threadIdx.x; i < k / 4; i += blockDim.x) {
-        const float4 v = reinterpret_cast<const float4 *>(xr)[i];
-        const double a = v.x, b = v.y, c = v.z, d = v.w;
-        sq[i] = a * a;
-        sq[cs + i] = b * b;
-        sq[2 * cs + i] = c * c;
-        sq[3 * cs + i] = d * d;
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        const float sc = rms_scale_wave(sq, k, eps);
-        if (threadIdx.x == 0) scale = sc;
-    }
-    __syncthreads();
-    const float sc = scale;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-        float xv[32], wv[32], v[32];
-        load_block(xr + 32 * b, xv);
-        load_block(w + 32 * b, wv);
+    float4 xv[NV], wv[NV];
 #pragma unroll
-        for (int e = 0; e < 32; ++e) {
-            const float a = xv[e] * sc;
-            v[e] = a * wv[e];
+    for (int j = 0; j < NV; ++j) {
+        const int i = threadIdx.x + 256 * j;       // n4 % 64 == 0: waves are in or out as a whole
+        const int c = i < n4 ? i : 0;
+        xv[j] = reinterpret_cast<const float4 *>(xr)[c];
+        wv[j] = reinterpret_cast<const float4 *>(w)[c];
+    }
+    double p = 0.0;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        if (threadIdx.x + 256 * j < n4) {
+            const double a = xv[j].x, b = xv[j].y, c = xv[j].z, d = xv[j].w;
+            p = fma(a, a, p);
+            p = fma(b, b, p);
+            p = fma(c, c, p);
+            p = fma(d, d, p);
         }
-        quantize_store<X_ENGINE>(v, row, b, k, out);
+    }
+    const float sc = rms_scale_block(p, k, eps, 4, part, [&](int i) { return xr[i]; });
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = threadIdx.x + 256 * j;
+        if (i < n4) {
+            const float4 v = make_float4((xv[j].x * sc) * wv[j].x, (xv[j].y * sc) * wv[j].y, (xv[j].z * sc) * wv[j].z,
+                                         (xv[j].w * sc) * wv[j].w);
+            quantize_store8<X_ENGINE>(v, row, i >> 3, i & 7, k, out);
+        }
     }
 }
 
@@ -221,10 +188,13 @@ hipError_t launch_silu_mul_q8_0(const float *gate_up, int k, int m, uint8_t *out
 hipError_t launch_rmsnorm_q8_0(const float *x, const float *w, float eps, int k, int m, uint8_t *out,
                                hipStream_t stream) {
     if (m <= 0) return hipSuccess;
-    const size_t lds = rms_sq_doubles(k) * 8;               // float64 squares: 128 KB at k = 16384
-    const hipError_t e = allow_dynamic_lds(reinterpret_cast<const void *>(&rmsnorm_q8_0_kernel), 160 * 1024);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(rmsnorm_q8_0_kernel, dim3((unsigned)m), dim3(256), lds, stream, x, w, eps, k, out);
+    // The float4s a thread holds: k / 1024, rounded up to a power of two.
+    auto *kernel = k <= 1024   ? &rmsnorm_q8_0_kernel<1>
+                   : k <= 2048 ? &rmsnorm_q8_0_kernel<2>
+                   : k <= 4096 ? &rmsnorm_q8_0_kernel<4>
+                   : k <= 8192 ? &rmsnorm_q8_0_kernel<8>
+                               : &rmsnorm_q8_0_kernel<16>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)m), dim3(256), 0, stream, x, w, eps, k, out);
     return hipGetLastError();
 }
 

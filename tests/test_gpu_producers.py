@@ -52,6 +52,49 @@ def test_silu_mul_q8_0(gpu, k, m):
     assert_bytes_equal(got, want, "silu_mul_q8_0")
 
 
+def _scale(mean, eps):
+    return np.float32(1) / np.sqrt(np.float32(mean) + np.float32(eps))
+
+
+def _mean_at_midpoint(k, kind, eps):
+    """x and norm weight whose mean square lies where the float32 rounding of
+    ss / n turns on the chains' order, and whose Q8_0 bytes tell the two
+    roundings apart (k a power of two; any other k is an ordinary row)."""
+    x, w = np.zeros(k, np.float32), np.ones(k, np.float32)
+    if kind == "overflow":                   # ss / n rounds to an infinity: the scale is 0
+        x[:] = 3e38
+        return x, w
+    for x0 in 1.0 + np.arange(1, 80) / 256:  # x0 * x0 + 1/4 < 2: a few bits, so that ss is exact but for the small squares
+        down = np.float32((x0 * x0 + 0.25) / k)
+        up = np.nextafter(down, np.float32(1))
+        if _scale(down, eps) != _scale(up, eps):
+            break
+    x[0], x[4], x[1] = x0, 0.5, 2.0 ** -12   # ss / n = down + half an ulp: rounded to even
+    if kind != "tie":                        # chain 0 loses each 2^-56 beside x0 * x0; chain 2 keeps their sum
+        x[8::4] = 2.0 ** -28
+    if kind == "kept":
+        x[2::4], x[8::4] = 2.0 ** -28, 0.0
+    if k & (k - 1) == 0:
+        c = (1.0 + np.arange(1 << 23) / 2.0 ** 23).astype(np.float32)
+        d = [(np.float32(x0) * _scale(m, eps) * c / np.float32(127)).astype(np.float16) for m in (down, up)]
+        w[0] = c[np.flatnonzero(d[0] != d[1])[0]]
+    return x, w
+
+
+@pytest.mark.parametrize("kind", ["tie", "lost", "kept", "overflow"])
+@pytest.mark.parametrize("k", [256, 1024, 2048, 3072, 4096, 8192, 16384])
+def test_rmsnorm_mean_between_floats(gpu, k, kind):
+    eps = 1e-12
+    x, w = _mean_at_midpoint(k, kind, eps)
+    h = C.rmsnorm(x, w, eps)
+    got = host(gpu.rmsnorm_q8_0_engine(dev(np.stack([x, x])), dev(w), eps))
+    assert_bytes_equal(got, np.stack([_engine(h)] * 2), f"rmsnorm_q8_0 {k} {kind}")
+    if k <= 8192:
+        blocks = C.quantize_q4_0(O.normal_f32((24, k), 71, 0.02))
+        y = host(gpu.gemv_rmsnorm(dev(blocks), k, dev(x), dev(w), eps))
+        assert_bytes_equal(y, C.gemv_q4_0(blocks, k, *C.quantize_q8_0(h)), f"gemv_rmsnorm {k} {kind}")
+
+
 @pytest.mark.parametrize("rows,k", [(3072, 2048), (100, 256), (512, 8192), (16384, 2048), (40, 768), (1024, 4096),
                                     (64, 2048), (136, 2048)])
 def test_gemv_rmsnorm(gpu, rows, k):
