@@ -53,9 +53,9 @@
 // Workgroups are persistent over items; a workgroup's rounds form one stream
 // that runs on across its items.
 //
-// Matrices of 8,192 rows and more go to gemm_rows.hip instead, which cuts the
-// work along rows (two or four waves per 16-row group for the whole of K):
-// with that many rows it fills the GPU without splitting K, and is faster.
+// Matrices of 8,192 rows and more go to gemm_rows.hip up to 16 tokens, which
+// cuts the work along rows (two or four waves per 16-row group for the whole
+// of K), and larger products of rows and tokens to gemm_tiles.hip.
 #include "kernels.h"
 #include "q4_0_device.h"
 
@@ -485,26 +485,24 @@ hipError_t launch_mt(const GemmParams &Pm, hipStream_t stream) {
     return launch_geo<MT, 1, OCC, NRL>(Pm, stream);
 }
 
-// Workgroups per CU, and the item count under which wide token tiles split
-// into 16-token items (below).
+// Workgroups per CU, and the item count under which 32-token tiles split into
+// 16-token items (below).
 constexpr int GEMM_OCC = 2;
 constexpr long GEMM_SPLIT_ITEMS = 160;
 
 hipError_t launch_tokens(const GemmParams &Pm, hipStream_t stream) {
-    // 16, 32 or 64 tokens per item. The widest tile that covers M streams the
-    // weights once. With few row groups (2,048 rows: o, down) that leaves
-    // most CUs idle, and 16-token items, one per (row group, token group),
-    // are faster: down at M = 64 in 16.9 us against 28.3, at M = 24 in 11.4
-    // against 16.2 (the weights are read once per token group, the later reads
-    // mostly from the caches). At 3,072 rows (192 row groups) 16-token items
-    // win at M > 32 only (8.8 against 9.5 us at M = 64; at M = 24 the 32-token
-    // tile is faster). A round holds 128 (or, at two workgroups per CU, 64)
-    // token-chunks of activations.
+    // 16 or 32 tokens per item. With few row groups (2,048 rows: o, down)
+    // 32-token items leave most CUs idle, and 16-token items, one per (row
+    // group, token group), are faster: down at M = 64 in 16.9 us against
+    // 28.3, at M = 24 in 11.4 against 16.2 (the weights are read once per
+    // token group, the later reads mostly from the caches). At 3,072 rows
+    // (192 row groups) and M = 24 the 32-token tile is faster. A round holds
+    // 128 (or, at two workgroups per CU, 64) token-chunks of activations.
     constexpr int OCC = GEMM_OCC;
     const long row_groups = (Pm.rows + NR - 1) / NR;
-    int mt = Pm.m <= 16 ? 1 : Pm.m <= 32 ? 2 : 4;
+    int mt = Pm.m <= 16 ? 1 : 2;
     const long wide_items = row_groups * ((Pm.m + 16 * mt - 1) / (16 * mt));
-    if (mt > 1 && (wide_items < GEMM_SPLIT_ITEMS || (mt == 4 && wide_items < 2 * GEMM_SPLIT_ITEMS))) mt = 1;
+    if (mt > 1 && wide_items < GEMM_SPLIT_ITEMS) mt = 1;
     // One token group over long rows (K >= 8192: down) with fewer 16-row
     // groups than CUs: 8-row items, eight chunks per round, one workgroup per
     // CU. Down at M = 5..16 takes 9.2-10.1 us against 10.4-10.6 with 16-row
@@ -514,15 +512,20 @@ hipError_t launch_tokens(const GemmParams &Pm, hipStream_t stream) {
     if (mt == 1 && Pm.m <= 16 && Pm.k >= 8192 && row_groups < device_cu_count())
         return launch_mt<1, 8, 1, 8>(Pm, stream);
     if (mt == 1) return launch_mt<1, 8 / OCC, OCC>(Pm, stream);
-    if (mt == 2) return launch_mt<2, 4 / OCC, OCC>(Pm, stream);
-    return launch_mt<4, 2 / OCC, OCC>(Pm, stream);
+    return launch_mt<2, 4 / OCC, OCC>(Pm, stream);
 }
 
 }  // namespace
 
-// From this many rows on, the row-split kernel: at gate|up (16,384 rows) it is
-// 8-26% faster; at 3,072 rows it was twice as slow (48 workgroups).
+// From this many rows on, the row-split kernel up to 16 tokens and the
+// whole-prompt kernel (gemm_tiles.hip) past that: at 8192 x 2048 6.6 against
+// 8.3 us at 16 tokens, 9.3 against 8.3 at 17; gate|up 7.9 and 9.0 at 16, 10.2
+// and 9.5 at 24; the LM head 47 and 59 at 16, 80 and 51 at 17. (Its kernels
+// for 17 to 64 tokens, now gone, took 14.9 us at gate|up and 64 tokens against
+// 13.3.) At 3,072 rows the row-split kernel was twice as slow as this file's
+// (48 workgroups).
 constexpr int ROWS_MIN = 8192;
+constexpr int ROWS_MAX_M = 16;
 
 hipError_t launch_gemm(const MatrixRef &w, const uint8_t *x, int m, float *y, hipStream_t stream) {
     // One token is the M = 1 GEMV, byte for byte by the contract, and faster.
@@ -539,21 +542,19 @@ hipError_t launch_gemm(const MatrixRef &w, const uint8_t *x, int m, float *y, hi
     P.rows = w.rows;
     P.k = w.k;
     P.x_stride = w.k + w.k / 8;
-    // Buffer ranges are 32-bit byte counts: the weights must fit one. Tokens
-    // go in launches of at most 64 (one item's tokens, so the weights stream
-    // once per launch), whose activations and outputs then fit one too.
+    P.x = x;
+    P.y = y;
+    P.m = m;
+    // Buffer ranges are 32-bit byte counts: the weights must fit one (and 64
+    // tokens' outputs, the limit these calls have always had).
     if ((size_t)P.rows * (size_t)(P.k / QK * Q4_0_BYTES) >= 0x7fff0000u ||
         (size_t)64 * P.rows * 4 >= 0x7fff0000u)
         return hipErrorInvalidValue;
     const bool by_rows = P.rows >= ROWS_MIN && gemm_rows_fits(P.rows, P.k);
-    for (int m0 = 0; m0 < m; m0 += 64) {
-        P.x = x + (size_t)m0 * P.x_stride;
-        P.y = y + (size_t)m0 * P.rows;
-        P.m = m - m0 < 64 ? m - m0 : 64;
-        const hipError_t e = by_rows ? launch_gemm_rows(P.w, P.x, P.m, P.y, P.rows, P.k, stream) : launch_tokens(P, stream);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    if (by_rows ? m > ROWS_MAX_M : gemm_tiles_faster(m, P.rows, P.k))
+        return launch_gemm_tiles(P.w, x, m, y, P.rows, P.k, stream);
+    if (by_rows) return launch_gemm_rows(P.w, x, m, y, P.rows, P.k, stream);
+    return launch_tokens(P, stream);   // rows * m below gemm_tiles_faster's line: the outputs fit a range too
 }
 
 }  // namespace w4a8

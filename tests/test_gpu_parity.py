@@ -331,6 +331,35 @@ def test_gemm_random_bytes(gpu, m, rows, k):
     assert_bytes_equal(host(y), want, "gemm, random bytes")
 
 
+@pytest.mark.parametrize("m,rows,k", [
+    (65, 700, 256), (1100, 128, 256),       # one chunk; many 32-token groups of few rows
+    (33, 1400, 768), (129, 1601, 768),      # odd chunk counts, a last group of one token, of one row
+    (96, 2305, 512), (97, 2309, 1024),      # whole 32-token groups, one token more
+    (17, 8200, 512), (6, 8300, 768),        # many rows, few tokens
+    (40, 8200, 512), (70, 8200, 256),       # 64-token tiles: 40 of 64, a last group of 6
+    (64, 16400, 256), (128, 8192, 2048)])
+def test_gemm_whole_prompt(gpu, m, rows, k):
+    rng = np.random.default_rng(m + rows)
+    w = (rng.standard_normal((rows, k)) * 0.02).astype(np.float32)
+    blocks = C.quantize_q4_0(w).reshape(rows, k // 32, 18)
+    blocks[rows // 2, 0, :2] = np.array([65504.0], np.float16).view(np.uint8)   # the largest finite scale
+    blocks[rows // 3, -1, :2] = np.array([-6e-8], np.float16).view(np.uint8)    # the smallest
+    blocks[rows - 1, 1, :2] = np.array([np.inf], np.float16).view(np.uint8)
+    blocks[0, 2, :2] = np.array([np.nan], np.float16).view(np.uint8)
+    blocks = blocks.reshape(rows, -1)
+    xq, xd = C.quantize_q8_0_rows((rng.standard_normal((m, k)) * 3).astype(np.float32))
+    xq, xd = xq.copy(), xd.copy()
+    xq[m - 1, :64] = -128                        # a caller's own int8: the largest sums
+    xd[m // 2, 3] = np.float16(np.inf)
+    want = C.gemm_q4_0_rows(blocks, k, xq, xd)
+    x_rows = np.stack([C.pack_x_for_engine(xq[i], xd[i]) for i in range(m)])
+    y = poisoned_f32((m + 1, rows))
+    gpu.gemm_engine(dev(blocks), k, dev(x_rows), out=y)
+    got = host(y)
+    assert_bytes_equal(got[:m], want, f"gemm {m}x{rows}x{k}")
+    assert (got[m].view(np.uint8) == 0xAA).all(), "written past the last token"
+
+
 def test_gemm_one_row_equals_gemv(gpu):
     rows, k = 96, 2048
     _, _, blocks, xq, xd = _case(rows, k, 130, 131)
