@@ -16,10 +16,18 @@
 // keys, four per lane as four lists of 64 (one key per lane each), sorts the
 // four across its lanes (bitonic, register compare-exchanges with the lane
 // `stride` apart), and merges them two by two; the four waves' best 64 then
-// merge through LDS, and the workgroup writes its 64 best. Stage 2: one
-// workgroup merges those lists pairwise, level by level. A merge of two
+// merge through LDS, and the workgroup writes its 64 best. A merge of two
 // descending lists A and B keeps, in lane l, max(A[l], B[63 - l]): a bitonic
 // sequence holding their 64 best, which six compare-exchange steps sort.
+//
+// Stage 2: one workgroup, so all of it is latency (a chain of shuffles,
+// barriers and loads), and it sorts as little as it can. With at least k
+// lists, the k-th largest list head is a bound no larger than the k-th best
+// key: the heads are sorted first (two to four lists of 64), the keys at or
+// above the bound gathered (about k of them for random logits), and up to 256
+// of them sorted and merged. More, or fewer lists than k, take the merge of
+// all lists pairwise, level by level. 128,256 logits, a call of both stages:
+// 14.4 us with the pairwise merge and shuffles through LDS, 12.5 so.
 //
 // A NaN logit has no place in that order: the reference's loop admits it
 // (v <= NaN is false) into the last slot, evicting the k-th candidate it
@@ -42,7 +50,9 @@ namespace {
 constexpr int TOPK_SLICE = 1024;      // logits per stage-1 workgroup
 constexpr int TOPK_LIST = 64;         // candidates each list keeps (k <= 64)
 constexpr int TOPK_MAX_LISTS = 256;   // stage 2's LDS: 256 x 64 keys = 128 KB
-static_assert(TOPK_LIST == 64, "the index arithmetic below takes lists of 64");
+constexpr int TOPK_CAND = 256;        // keys stage 2 sorts without the pairwise merge (and list heads)
+static_assert(TOPK_LIST == 64 && TOPK_CAND == 4 * TOPK_LIST && TOPK_CAND >= TOPK_MAX_LISTS,
+              "the index arithmetic below takes lists of 64, four of them in `cand`");
 
 constexpr unsigned long long NAN_MARK = ~0ull;   // a stage-1 list whose slice holds a NaN
 
@@ -55,16 +65,34 @@ __device__ __forceinline__ unsigned long long topk_key(float v, int i) {
 
 __device__ __forceinline__ unsigned long long max_u64(unsigned long long a, unsigned long long b) { return a > b ? a : b; }
 
-// The value of lane l ^ S for one 32-bit word: DPP for S = 1, 2, 8 (quad
-// permutations, a rotation by 8 within a row of 16), an LDS swizzle in
-// bit mode for S = 4, 16, ds_bpermute for S = 32.
+// The value of lane l ^ S for one 32-bit word, all in the VALU (through LDS, a
+// swizzle or ds_bpermute takes some 60 clocks, and a sort is a chain of them):
+// DPP for S = 1, 2, 8 (quad permutations, a rotation by 8 within a row of 16),
+// two for S = 4 (mirror the half row, then the quads: l ^ 7 ^ 3), the row and
+// half swaps for S = 16, 32 (of a register with itself: one result holds the
+// even rows twice, or the lower half, the other the odd ones).
 template <int S>
 __device__ __forceinline__ int xor_lane(int v, int lane) {
     if constexpr (S == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
     else if constexpr (S == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
     else if constexpr (S == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false);  // row_ror:8
-    else if constexpr (S == 4 || S == 16) return __builtin_amdgcn_ds_swizzle(v, (S << 10) | 0x1F);
-    else return __builtin_amdgcn_ds_bpermute((lane ^ S) << 2, v);
+    else if constexpr (S == 4)   // row_half_mirror, quad_perm [3,2,1,0]
+        return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, false), 0x1B, 0xF, 0xF, false);
+    else if constexpr (S == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+        return (int)((lane & 16) ? r[0] : r[1]);
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+        return (int)((lane & 32) ? r[0] : r[1]);
+    }
+}
+
+// The list read backwards: lane l gets lane 63 - l's key.
+__device__ __forceinline__ unsigned long long reversed(unsigned long long v, int lane) {
+    auto word = [&](int w) {
+        return (uint32_t)xor_lane<32>(xor_lane<16>(__builtin_amdgcn_mov_dpp(w, 0x140, 0xF, 0xF, false), lane), lane);   // row_mirror
+    };
+    return ((unsigned long long)word((int)(uint32_t)(v >> 32)) << 32) | word((int)(uint32_t)v);
 }
 
 // One compare-exchange step of a bitonic network over the wave's 64 lanes:
@@ -122,14 +150,14 @@ __global__ __launch_bounds__(256) void topk_stage1(const float *__restrict__ y, 
     bool nan = false;
 #pragma unroll
     for (int r = 0; r < 4; ++r) nan = nan || (base + 64 * r + lane < n && v[r] != v[r]);
-    const unsigned long long m01 = merge64(k[0], __shfl(k[1], 63 - lane), lane);
-    const unsigned long long m23 = merge64(k[2], __shfl(k[3], 63 - lane), lane);
-    wl[wave][lane] = merge64(m01, __shfl(m23, 63 - lane), lane);
+    const unsigned long long m01 = merge64(k[0], reversed(k[1], lane), lane);
+    const unsigned long long m23 = merge64(k[2], reversed(k[3], lane), lane);
+    wl[wave][lane] = merge64(m01, reversed(m23, lane), lane);
     const bool slice_has_nan = __syncthreads_or(nan);
     if (wave == 0) {
         const unsigned long long a = merge64(wl[0][lane], wl[1][63 - lane], lane);
         const unsigned long long b = merge64(wl[2][lane], wl[3][63 - lane], lane);
-        const unsigned long long best = merge64(a, __shfl(b, 63 - lane), lane);
+        const unsigned long long best = merge64(a, reversed(b, lane), lane);
         lists[(size_t)blockIdx.x * TOPK_LIST + lane] = slice_has_nan && lane == 0 ? NAN_MARK : best;
     }
 }
@@ -192,49 +220,107 @@ __global__ __launch_bounds__(1024) void topk_stage2(const float *__restrict__ y,
                                                     float *__restrict__ vals,
                                                     int32_t *__restrict__ idx) {
     extern __shared__ __attribute__((aligned(16))) unsigned long long lk[];
+    __shared__ unsigned long long cand[TOPK_CAND];
+    __shared__ int n_cand;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (__syncthreads_or(t < nlists && lists[(size_t)t * TOPK_LIST] == NAN_MARK)) {
+    // Up to 16 keys per thread (256 lists of 64), all loaded before any is
+    // used: key j is place `lane` of list 16 j + wave; missing lists are empty
+    // (key 0).
+    constexpr int KEYS = TOPK_MAX_LISTS * TOPK_LIST / 1024;
+    const int have = nlists * TOPK_LIST;
+    const unsigned long long head = lists[(size_t)(t < nlists ? t : 0) * TOPK_LIST];
+    unsigned long long kv[KEYS];
+#pragma unroll
+    for (int j = 0; j < KEYS; ++j) {
+        const int i = t + 1024 * j;
+        kv[j] = lists[i < have ? i : have - 1];
+    }
+    // Four waves sort the heads, 64 each.
+    if (t < TOPK_CAND) cand[t] = sort64(t < nlists ? head : 0ull, lane);
+    if (t == 0) n_cand = 0;
+    if (__syncthreads_or(t < nlists && head == NAN_MARK)) {
         if (wave == 0) topk_in_order(y, n, k, vals, idx, lane);
         return;
     }
-    int np = 1;
-    while (np < nlists) np <<= 1;
-    {
-        // Up to 16 keys per thread (256 lists of 64), all loaded before any
-        // is stored; missing lists are empty (key 0).
-        const int have = nlists * TOPK_LIST;
-        unsigned long long kv[TOPK_MAX_LISTS * TOPK_LIST / 1024];
 #pragma unroll
-        for (int j = 0; j < TOPK_MAX_LISTS * TOPK_LIST / 1024; ++j) {
-            const int i = t + 1024 * j;
-            kv[j] = lists[i < have ? i : have - 1];
-        }
+    for (int j = 0; j < KEYS; ++j)
+        if (t + 1024 * j >= have) kv[j] = 0ull;
+    // The 64 best of four sorted lists in `cand`, in every wave.
+    auto best_of_four = [&]() {
+        const unsigned long long a = merge64(cand[lane], cand[127 - lane], lane);
+        const unsigned long long b = merge64(cand[128 + lane], cand[255 - lane], lane);
+        return merge64(a, reversed(b, lane), lane);
+    };
+    bool done = false;
+    unsigned long long out = 0ull;
+    if (nlists >= k) {
+        const unsigned long long heads = best_of_four();
+        // The k-th largest head (k <= nlists: it is a list's, and 0 only if
+        // that list is empty). Keys differ, so k keys at least reach it.
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)heads, k - 1);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(heads >> 32), k - 1);
+        const unsigned long long bound = max_u64(((unsigned long long)hi << 32) | lo, 1ull);
+        // Each list's keys at or above the bound are its first ones.
+        int count = 0;
 #pragma unroll
-        for (int j = 0; j < TOPK_MAX_LISTS * TOPK_LIST / 1024; ++j) {
-            const int i = t + 1024 * j;
-            if (i < np * TOPK_LIST) lk[i] = i < have ? kv[j] : 0ull;
+        for (int j = 0; j < KEYS; ++j) count += __builtin_popcountll(__ballot(kv[j] >= bound));
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&n_cand, count);
+        at = __builtin_amdgcn_readfirstlane(at);
+        __syncthreads();                          // the heads are read in every wave, the count is whole
+        const int total = n_cand;
+        done = total <= TOPK_CAND;
+        if (done) {
+#pragma unroll
+            for (int j = 0; j < KEYS; ++j) {
+                const unsigned long long m = __ballot(kv[j] >= bound);
+                if (kv[j] >= bound) cand[at + lane] = kv[j];
+                at += __builtin_popcountll(m);
+            }
+            if (t >= total && t < TOPK_CAND) cand[t] = 0ull;
+            __syncthreads();
+            if (total <= TOPK_LIST) {
+                if (wave == 0) out = sort64(cand[lane], lane);
+            } else {
+                unsigned long long v = 0ull;
+                if (t < TOPK_CAND) v = sort64(cand[t], lane);
+                if (t < TOPK_CAND) cand[t] = v;
+                __syncthreads();
+                if (wave == 0) out = best_of_four();
+            }
         }
     }
-    // Level by level: lists a = 2 g s and b = a + s meet into a, a wave per pair.
-    for (int s = 1; s < np; s <<= 1) {
+    if (!done) {
+        int np = 1;
+        while (np < nlists) np <<= 1;
+#pragma unroll
+        for (int j = 0; j < KEYS; ++j) {
+            const int i = t + 1024 * j;
+            if (i < np * TOPK_LIST) lk[i] = kv[j];
+        }
+        // Level by level: lists a = 2 g s and b = a + s meet into a, a wave per pair.
+        for (int s = 1; s < np; s <<= 1) {
+            __syncthreads();
+            const int pairs = np / (2 * s);
+            for (int g = wave; g < pairs; g += 16) {
+                unsigned long long *a = lk + (size_t)(2 * g * s) * TOPK_LIST;
+                const unsigned long long *b = a + (size_t)s * TOPK_LIST;
+                const unsigned long long m = merge64(a[lane], b[63 - lane], lane);
+                a[lane] = m;
+            }
+        }
         __syncthreads();
-        const int pairs = np / (2 * s);
-        for (int g = wave; g < pairs; g += 16) {
-            unsigned long long *a = lk + (size_t)(2 * g * s) * TOPK_LIST;
-            const unsigned long long *b = a + (size_t)s * TOPK_LIST;
-            const unsigned long long m = merge64(a[lane], b[63 - lane], lane);
-            a[lane] = m;
-        }
+        if (wave == 0) out = lk[lane];
     }
-    __syncthreads();
     if (t < k) {
-        const unsigned long long key = lk[t];
-        if (key == 0ull) {
+        if (out == 0ull) {
             vals[t] = -1e30f;
             idx[t] = 0;
         } else {
-            const int i = (int)(0xFFFFFFFFu - (uint32_t)key);
-            vals[t] = y[i];
+            // The value back from its order bits; a zero's sign is y's.
+            const int i = (int)(0xFFFFFFFFu - (uint32_t)out);
+            const uint32_t ord = (uint32_t)(out >> 32);
+            vals[t] = ord == 0x80000000u ? y[i] : __uint_as_float((ord & 0x80000000u) ? ord & 0x7FFFFFFFu : ~ord);
             idx[t] = i;
         }
     }
@@ -295,8 +381,7 @@ hipError_t launch_topk(const float *y, int n, int k, float *vals, int32_t *idx, 
     const int nlists = (n + TOPK_SLICE - 1) / TOPK_SLICE;
     if (n < 1 || nlists > TOPK_MAX_LISTS || k < 1 || k > TOPK_LIST) return hipErrorInvalidValue;
     auto *lists = static_cast<unsigned long long *>(workspace);
-    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void *>(&topk_stage2),
-                                     (size_t)TOPK_MAX_LISTS * TOPK_LIST * sizeof(unsigned long long));
+    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void *>(&topk_stage2), 160 * 1024);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(topk_stage1, dim3((unsigned)nlists), dim3(256), 0, stream, y, n, lists);
     e = hipGetLastError();

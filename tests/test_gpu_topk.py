@@ -59,6 +59,30 @@ def test_special_values(gpu):
     _check(gpu, np.zeros(4096, dtype=np.float32), 64, "all zero")
 
 
+@pytest.mark.parametrize("n,k", [(65536, 64), (65536 - 1024, 64), (8192, 8), (8192, 9), (262144, 64), (262143, 40)])
+@pytest.mark.parametrize("how", ["one slice", "few slices", "every slice", "descending", "negative zeros"])
+def test_topk_where_the_best_lie(gpu, n, k, how):
+    """Lists (1,024 logits each) as many as k and one fewer or more, and candidates at or above
+    the k-th list head from one list's 64 up to more than the 256 that are sorted by themselves."""
+    y = _logits(n, n + k)
+    rng = np.random.default_rng(k)
+    if how == "one slice":
+        y[n - 900:n - 700] += 100.0
+    elif how == "few slices":               # 64 in each of k / 2 slices: past 256
+        for c in range(max(k // 2, 1)):
+            y[1024 * c:1024 * c + 64] += 50.0 + rng.standard_normal(64).astype(np.float32)
+    elif how == "every slice":              # each slice a full list above the rest
+        for c in range(n // 1024):
+            y[1024 * c + 100:1024 * c + 164] += 50.0
+    elif how == "descending":
+        y = np.sort(y)[::-1].copy()
+    else:                                   # ties of +0 and -0, their bits kept
+        y = -np.abs(y)
+        at = rng.choice(n, 200, replace=False)
+        y[at] = np.where(np.arange(200) % 2, F32(0.0), F32(-0.0))
+    _check(gpu, y, k, f"n={n} k={k} {how}")
+
+
 def test_first_candidate_is_the_fused_argmax(gpu):
     import q4_0_oracle as O
     rows, k = 128256, 2048
