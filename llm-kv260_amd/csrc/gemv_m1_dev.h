@@ -363,11 +363,22 @@ __device__ __forceinline__ void gemv_m1_body(const GemvParams &P, int block, int
     [[maybe_unused]] XLines xl;
     const bool lines = XF == X_F32 && nthreads >= nb;
     const bool x_wave = __builtin_amdgcn_readfirstlane(wave) * 64 < nb;
+    // ARGMAX (the LM head, several tiles a wave): the norm weight goes out
+    // after the first tile. Its address is not among the preloaded arguments,
+    // and ahead of the tile it holds the tile back for its argument's fetch:
+    // 26.5 -> 26.4 us. With one tile a wave it comes too late behind it (the
+    // fused decode step 294 us against 275).
+    auto load_norm = [&]() {
+        if constexpr (XF == X_RMS) {
+            if (quarter) norm_load_quarter(P.norm_w, P.k, tid >> 2, tid & 3, tid < 4 * nb, xq);
+        }
+    };
     auto load_x = [&]() {
         if constexpr (XF == X_RMS) {
-            if (quarter)
-                x_load_quarter<XAUX>(P.x, P.norm_w, P.k, tid >> 2, tid & 3, tid < 4 * nb, xq);
-            else
+            if (quarter) {
+                x_load_quarter<XAUX>(P.x, P.k, tid >> 2, tid & 3, tid < 4 * nb, xq);
+                if constexpr (!ARGMAX) load_norm();
+            } else
                 x_load<XF, XAUX>(P.x, P.k, tid, tid < nb, xr, P.norm_w);
         } else if constexpr (XF == X_F32) {
             if (lines) {
@@ -580,7 +591,10 @@ __device__ __forceinline__ void gemv_m1_body(const GemvParams &P, int block, int
     if (n_my >= 2) {
         Tile buf[DEPTH];
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) load_tile<PLAIN>(P, tile + d * tstride, lane, buf[d]);
+        for (int d = 0; d < DEPTH; ++d) {
+            load_tile<PLAIN>(P, tile + d * tstride, lane, buf[d]);
+            if (ARGMAX && d == 0) load_norm();
+        }
         after_weights();
         stage_x();
         int done = 0;
@@ -593,11 +607,13 @@ __device__ __forceinline__ void gemv_m1_body(const GemvParams &P, int block, int
             if (done + d < n_my) step(buf[d], last_t{});
     } else if (n_my == 1) {
         Tile b;
+        if constexpr (ARGMAX) load_norm();
         load_tile<PLAIN>(P, tile, lane, b);
         after_weights();
         stage_x();
         step(b, last_t{});
     } else {
+        if constexpr (ARGMAX) load_norm();
         after_weights();
         stage_x();
     }

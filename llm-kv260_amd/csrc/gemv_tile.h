@@ -3,6 +3,8 @@
 // one chunk, and the contract's ordered lane sums.
 #pragma once
 
+#include <type_traits>
+
 #include "kernels.h"
 #include "q4_0_device.h"
 
@@ -163,18 +165,21 @@ struct XQuarter {
     float4 xa, xb, wa, wb;
 };
 
-template <int AUX = 0>
-__device__ __forceinline__ void x_load_quarter(const void *x, const float *norm_w, int k, int b, int q, bool live,
-                                               XQuarter &r) {
-    const __amdgpu_buffer_rsrc_t xr = buffer_of(x, (uint32_t)(4 * k));
-    const __amdgpu_buffer_rsrc_t wr = buffer_of(norm_w, (uint32_t)(4 * k));
-    const int off = live ? 128 * b + 16 * q : OUT_OF_RANGE;
-    const int off2 = live ? off + 64 : OUT_OF_RANGE;
+template <class Aux>
+__device__ __forceinline__ void load_quarter(__amdgpu_buffer_rsrc_t rsrc, int off, float4 &a, float4 &b, Aux) {
+    const int off2 = off == OUT_OF_RANGE ? OUT_OF_RANGE : off + 64;
     auto f4 = [](u32x4 t) { return make_float4(__uint_as_float(t.x), __uint_as_float(t.y), __uint_as_float(t.z), __uint_as_float(t.w)); };
-    r.xa = f4(__builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, AUX));
-    r.xb = f4(__builtin_amdgcn_raw_buffer_load_b128(xr, off2, 0, AUX));
-    r.wa = f4(__builtin_amdgcn_raw_buffer_load_b128(wr, off, 0, 0));
-    r.wb = f4(__builtin_amdgcn_raw_buffer_load_b128(wr, off2, 0, 0));
+    a = f4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, Aux::value));
+    b = f4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, off2, 0, Aux::value));
+}
+template <int AUX = 0>
+__device__ __forceinline__ void x_load_quarter(const void *x, int k, int b, int q, bool live, XQuarter &r) {
+    load_quarter(buffer_of(x, (uint32_t)(4 * k)), live ? 128 * b + 16 * q : OUT_OF_RANGE, r.xa, r.xb,
+                 std::integral_constant<int, AUX>{});
+}
+__device__ __forceinline__ void norm_load_quarter(const float *norm_w, int k, int b, int q, bool live, XQuarter &r) {
+    load_quarter(buffer_of(norm_w, (uint32_t)(4 * k)), live ? 128 * b + 16 * q : OUT_OF_RANGE, r.wa, r.wb,
+                 std::integral_constant<int, 0>{});
 }
 
 // The rmsnorm block's staging by its four threads (lanes 4b' .. 4b' + 3 of a

@@ -337,7 +337,8 @@ def test_gemm_random_bytes(gpu, m, rows, k):
     (96, 2305, 512), (97, 2309, 1024),      # whole 32-token groups, one token more
     (17, 8200, 512), (6, 8300, 768),        # many rows, few tokens
     (40, 8200, 512), (70, 8200, 256),       # 64-token tiles: 40 of 64, a last group of 6
-    (64, 16400, 256), (128, 8192, 2048)])
+    (64, 16400, 256), (128, 8192, 2048),
+    (100, 700, 1024), (300, 100, 512), (70, 512, 3072)])   # the class-split kernel past 64 tokens
 def test_gemm_whole_prompt(gpu, m, rows, k):
     rng = np.random.default_rng(m + rows)
     w = (rng.standard_normal((rows, k)) * 0.02).astype(np.float32)
