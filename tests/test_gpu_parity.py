@@ -220,9 +220,8 @@ def test_gemv_nonfinite_scales(gpu):
                                     (24, 2000)])
 def test_gemm_nonfinite_scales(gpu, m, rows):
     """The M > 1 kernels with infinite and NaN fp16 scales, byte for byte, NaN outputs
-    included: the row-split kernels at every token tiling (8,200 rows: packed block pairs,
-    one, two and four token tiles), the few-token GEMV and the class-split kernel (2,000
-    rows)."""
+    included: the row-split kernels at 4 to 16 tokens and the whole-prompt kernel past them
+    (8,200 rows), the few-token GEMV and the class-split kernel (2,000 rows)."""
     rng = np.random.default_rng(190 + m)
     k = 1024
     blocks = C.quantize_q4_0(O.normal_f32((rows, k), 191, 0.02)).reshape(rows, k // 32, 18)
