@@ -56,6 +56,7 @@
 // Matrices of 8,192 rows and more go to gemm_rows.hip up to 16 tokens, which
 // cuts the work along rows (two or four waves per 16-row group for the whole
 // of K), and larger products of rows and tokens to gemm_tiles.hip.
+#include "gemm_route.h"
 #include "kernels.h"
 #include "q4_0_device.h"
 
@@ -485,24 +486,16 @@ hipError_t launch_mt(const GemmParams &Pm, hipStream_t stream) {
     return launch_geo<MT, 1, OCC, NRL>(Pm, stream);
 }
 
-// Workgroups per CU, and the item count under which 32-token tiles split into
-// 16-token items (below).
+// Workgroups per CU.
 constexpr int GEMM_OCC = 2;
-constexpr long GEMM_SPLIT_ITEMS = 160;
 
 hipError_t launch_tokens(const GemmParams &Pm, hipStream_t stream) {
-    // 16 or 32 tokens per item. With few row groups (2,048 rows: o, down)
-    // 32-token items leave most CUs idle, and 16-token items, one per (row
-    // group, token group), are faster: down at M = 64 in 16.9 us against
-    // 28.3, at M = 24 in 11.4 against 16.2 (the weights are read once per
-    // token group, the later reads mostly from the caches). At 3,072 rows
-    // (192 row groups) and M = 24 the 32-token tile is faster. A round holds
+    // 16 or 32 tokens per item. With several token groups the weights are read
+    // once per group, the later reads mostly from the caches. A round holds
     // 128 (or, at two workgroups per CU, 64) token-chunks of activations.
     constexpr int OCC = GEMM_OCC;
     const long row_groups = (Pm.rows + NR - 1) / NR;
-    int mt = Pm.m <= 16 ? 1 : 2;
-    const long wide_items = row_groups * ((Pm.m + 16 * mt - 1) / (16 * mt));
-    if (mt > 1 && wide_items < GEMM_SPLIT_ITEMS) mt = 1;
+    const int mt = gemm_route::split_tokens(Pm.m, Pm.rows, Pm.k, device_cu_count()) / 16;
     // One token group over long rows (K >= 8192: down) with fewer 16-row
     // groups than CUs: 8-row items, eight chunks per round, one workgroup per
     // CU. Down at M = 5..16 takes 9.2-10.1 us against 10.4-10.6 with 16-row

@@ -1,0 +1,39 @@
+// Which form an M > 1 product takes, from its sizes and the GPU's CU count.
+// Free of HIP types so that a CPU test (tests/test_gemm_route.py) holds the
+// rules against measured times.
+#pragma once
+
+namespace w4a8 {
+namespace gemm_route {
+
+// How many times the CUs are covered by the class-split kernel's items of 16
+// rows x `tokens` tokens (gemm_mfma.hip). Its time goes in such steps: a CU's
+// first item takes the latency of its rounds, each more about half of that.
+inline long covers(int m, int rows, int cus, int tokens) {
+    const long items = (long)((rows + 15) / 16) * ((m + tokens - 1) / tokens);
+    return (items + cus - 1) / cus;
+}
+
+// Tokens per item of the class-split kernel, 16 or 32, for the same launch. A
+// 32-token item takes 1.25 to 1.6 times a 16-token one's time.
+//  * Two covers of 16 against one of 32: 32 (3072 x 2048 at 24 tokens 6.7
+//    against 7.0 us, 3072 x 5888 17.1 against 21.6). But a round of a 16-token
+//    item is four chunks where k allows it, of a 32-token one two, so 16 keeps
+//    up on long rows: from k = 6144 it is up to 8% faster (2048 x 8192 at 33
+//    tokens 15.4 against 16.3) where its rounds are even in number (they go in
+//    pairs: at 7168 up to 6% slower). Past 64 tokens that starts at 8192 (900
+//    x 6144 at 128: 14.8 against 13.6).
+//  * As many covers of each, 16: 2560 x 8192 at 33 tokens 16.0 against 22.6.
+//  * One cover more of 16: 16 with rounds of four chunks (3072 x 2048 at 64
+//    tokens 8.3 against 9.4, 3072 x 8192 20.6 against 23.9), 32 where both
+//    have the same rounds (k no multiple of 1024; 3333 x 3584 at 48 tokens
+//    16.0 against 13.9). Two more, 32 (4096 x 8192 at 64 27.9 against 25.0).
+inline int split_tokens(int m, int rows, int k, int cus) {
+    const long n16 = covers(m, rows, cus, 16), n32 = covers(m, rows, cus, 32);
+    if (m <= 16 || n16 <= 1) return 16;
+    if (n32 == 1) return n16 == 2 && k >= (m > 64 ? 8192 : 6144) && k % 2048 == 0 ? 16 : 32;
+    return n16 <= n32 + (k % 1024 == 0) ? 16 : 32;
+}
+
+}  // namespace gemm_route
+}  // namespace w4a8
