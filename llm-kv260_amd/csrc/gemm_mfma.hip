@@ -544,10 +544,10 @@ hipError_t launch_gemm(const MatrixRef &w, const uint8_t *x, int m, float *y, hi
         (size_t)64 * P.rows * 4 >= 0x7fff0000u)
         return hipErrorInvalidValue;
     const bool by_rows = P.rows >= ROWS_MIN && gemm_rows_fits(P.rows, P.k);
-    if (by_rows ? m > ROWS_MAX_M : gemm_tiles_faster(m, P.rows, P.k))
+    if (by_rows ? m > ROWS_MAX_M : gemm_route::tiles_faster(m, P.rows, P.k, device_cu_count()))
         return launch_gemm_tiles(P.w, x, m, y, P.rows, P.k, stream);
     if (by_rows) return launch_gemm_rows(P.w, x, m, y, P.rows, P.k, stream);
-    return launch_tokens(P, stream);   // rows * m below gemm_tiles_faster's line: the outputs fit a range too
+    return launch_tokens(P, stream);   // at most two covers of 32-token items: the outputs fit a range too
 }
 
 }  // namespace w4a8

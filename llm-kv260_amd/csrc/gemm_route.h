@@ -35,5 +35,32 @@ inline int split_tokens(int m, int rows, int k, int cus) {
     return n16 <= n32 + (k % 1024 == 0) ? 16 : 32;
 }
 
+// Whether the whole-prompt kernel (gemm_tiles.hip) takes the product from the
+// class-split kernel. One of its launches is one cover up to 64 tokens x 64
+// rows a CU, at about 2.5 + 0.7 us a chunk: more than one or two of the
+// class-split kernel's covers, less than three.
+//  * Three covers of 32-token items and more: 2304 x 4096 at 160 tokens 15
+//    against 18 us, 3072 x 5888 at 130 20 against 43.
+//  * None of one cover (2048 x 8192 at 24 tokens 27 against 11), but for a
+//    single chunk, where no round's latency hides another's: 64 x 256 at 6
+//    tokens 3.1 against 3.4, 700 x 256 at 130 3.5 against 4.4; and past 64
+//    tokens where rounds are one chunk, from about 45,000 outputs on: 300 x
+//    1280 at 200 tokens 6.6 against 7.0, 16 x 2304 at 4,000 9.2 against 16.6
+//    (64 x 2304 at 300 8.8 against 8.1).
+//  * Two covers of 32, where rounds are one chunk (k no multiple of 512): 3333
+//    x 2304 at 48 tokens 9.6 against 12.1. Else only on short rows, the
+//    shorter the fewer 16-token items there are instead; up to 32 tokens on
+//    shorter ones still, the weights then being most of its time (7168 x 3072
+//    at 25 tokens 12.3 against 11.8, 3333 x 3072 at 72 11.7 against 15.4).
+inline bool tiles_faster(int m, int rows, int k, int cus) {
+    const long n16 = covers(m, rows, cus, 16), n32 = covers(m, rows, cus, 32);
+    if (k == 256 || n32 >= 3) return true;
+    if (n32 == 1) return k % 512 && m > 64 && (long)rows * m >= 45000;
+    if (k % 512) return true;
+    if (n16 == 2) return k < 1024;
+    if (m <= 32) return k < 2048;
+    return k < (n16 == 3 && k % 1024 == 0 ? 2048 : 4096);
+}
+
 }  // namespace gemm_route
 }  // namespace w4a8

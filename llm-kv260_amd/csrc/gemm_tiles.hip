@@ -418,16 +418,4 @@ hipError_t launch_gemm_tiles(const uint8_t *w, const uint8_t *x, int m, float *y
     return launch_tiles<4>(P, stream);
 }
 
-// Against the class-split kernel (gemm_mfma.hip). A launch of one tile a CU
-// takes about 2.5 + 0.66 us a chunk however small the matrix; the class-split
-// kernel about 3 us and 12 us for each 2^30 of rows * m * k (twice that where
-// k is no multiple of 512 and its rounds are one chunk). The lines cross at
-// the rows * m below: 3072 x 2048 at 64 tokens (197k) 8.4 us here, 8.3 there,
-// 4096 x 4096 at 64 (262k) 14.2 and 16.7, 2048 x 8192 at 64 (131k) 24 and 16,
-// 2304 x 5888 at 17 (39k) 18 and 21.
-bool gemm_tiles_faster(int m, int rows, int k) {
-    const long from = k % 512 ? 45000 : 220000 - 42600000 / k;
-    return (long)rows * m >= from;
-}
-
 }  // namespace w4a8
