@@ -494,15 +494,9 @@ hipError_t launch_tokens(const GemmParams &Pm, hipStream_t stream) {
     // once per group, the later reads mostly from the caches. A round holds
     // 128 (or, at two workgroups per CU, 64) token-chunks of activations.
     constexpr int OCC = GEMM_OCC;
-    const long row_groups = (Pm.rows + NR - 1) / NR;
-    const int mt = gemm_route::split_tokens(Pm.m, Pm.rows, Pm.k, device_cu_count()) / 16;
-    // One token group over long rows (K >= 8192: down) with fewer 16-row
-    // groups than CUs: 8-row items, eight chunks per round, one workgroup per
-    // CU. Down at M = 5..16 takes 9.2-10.1 us against 10.4-10.6 with 16-row
-    // items (MI355X, rotated weights). With several token groups (M > 16) a
-    // workgroup then runs its items one after another, 1.5-1.8x slower, and at
-    // K = 2048 (o, q|k|v) 8-row items were slower too.
-    if (mt == 1 && Pm.m <= 16 && Pm.k >= 8192 && row_groups < device_cu_count())
+    const int cus = device_cu_count();
+    const int mt = gemm_route::split_tokens(Pm.m, Pm.rows, Pm.k, cus) / 16;
+    if (gemm_route::split_rows(Pm.m, Pm.rows, Pm.k, cus) == 8)
         return launch_mt<1, 8, 1, 8>(Pm, stream);
     if (mt == 1) return launch_mt<1, 8 / OCC, OCC>(Pm, stream);
     return launch_mt<2, 4 / OCC, OCC>(Pm, stream);

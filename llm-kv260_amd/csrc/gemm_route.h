@@ -35,6 +35,16 @@ inline int split_tokens(int m, int rows, int k, int cus) {
     return n16 <= n32 + (k % 1024 == 0) ? 16 : 32;
 }
 
+// Rows per item of the class-split kernel for one token group, 16 or 8. Over
+// long rows (k >= 8192: down), while 8-row items cover the CUs once: eight
+// chunks a round, one workgroup a CU, 2048 x 8192 at 5 to 16 tokens in 9.2-10.1
+// us against 10.4-10.6. Past that a CU runs two of them one after the other
+// (3072 x 8192 at 16 16.3 against 10.6, 3072 x 16128 72 against 37), and at k =
+// 2048 (o, q|k|v) they were slower too.
+inline int split_rows(int m, int rows, int k, int cus) {
+    return m <= 16 && k >= 8192 && (rows + 7) / 8 <= cus ? 8 : 16;
+}
+
 // Whether the whole-prompt kernel (gemm_tiles.hip) takes the product from the
 // class-split kernel. One of its launches is one cover up to 64 tokens x 64
 // rows a CU, at about 2.5 + 0.7 us a chunk: more than one or two of the

@@ -9,7 +9,8 @@ using namespace w4a8;
 int main() {
     int m, rows, k, cus;
     while (std::scanf("%d %d %d %d", &m, &rows, &k, &cus) == 4)
-        std::printf("split%d %s\n", gemm_route::split_tokens(m, rows, k, cus),
+        std::printf("split%d rows%d %s\n", gemm_route::split_tokens(m, rows, k, cus),
+                    gemm_route::split_rows(m, rows, k, cus),
                     gemm_route::tiles_faster(m, rows, k, cus) ? "tiles" : "split");
     return 0;
 }

@@ -71,6 +71,13 @@ TIMES = (
     (17, 7168, 16384, 49.6, 41.6, 52.2),
 )
 
+# m, rows, k, then microseconds: 8-row and 16-row items of the class-split kernel.
+ROW_TIMES = (
+    (16, 2048, 8192, 10.1, 10.4), (16, 2064, 8192, 15.4, 10.3), (16, 2064, 8448, 39.7, 20.7),
+    (16, 2304, 16384, 27.6, 17.4), (16, 3072, 8192, 16.1, 10.5), (16, 4000, 11776, 34.1, 18.3),
+    (16, 4096, 8192, 16.2, 10.7),
+)
+
 
 def _covers(m, rows, tokens):
     return -(-(-(-rows // 16) * -(-m // tokens)) // CUS)
@@ -91,9 +98,10 @@ def routes(tmp_path_factory):
     def run(sizes):
         text = "".join(f"{m} {rows} {k} {CUS}\n" for m, rows, k in sizes)
         out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=60).stdout
-        # Per size: the class-split kernel's items and the form taken, as indices into a row's times.
-        return [(int(s == "split32"), 2 if f == "tiles" else int(s == "split32"))
-                for s, f in (line.split() for line in out.splitlines())]
+        # Per size: the class-split kernel's items and the form taken, as indices into a
+        # row's times, and its rows per item.
+        return [(int(s == "split32"), 2 if f == "tiles" else int(s == "split32"), int(r[4:]))
+                for s, r, f in (line.split() for line in out.splitlines())]
     return run
 
 
@@ -104,21 +112,26 @@ def _slow(times, chosen, forms=3):
 
 def test_items_of_the_class_split_kernel(routes):
     got = routes([t[:3] for t in SPLIT_TIMES])
-    assert not _slow(SPLIT_TIMES, [split for split, _ in got], 2)
+    assert not _slow(SPLIT_TIMES, [split for split, _, _ in got], 2)
 
 
 def test_form_taken(routes):
     got = routes([t[:3] for t in TIMES])
-    assert not _slow(TIMES, [form for _, form in got])
+    assert not _slow(TIMES, [form for _, form, _ in got])
 
 
 def test_line_in_rows_times_tokens_is_caught(routes):
     got = routes([t[:3] for t in TIMES])
     line = [2 if t[0] * t[1] >= (45000 if t[2] % 512 else 220000 - 42600000 // t[2]) else split
-            for t, (split, _) in zip(TIMES, got)]
+            for t, (split, _, _) in zip(TIMES, got)]
     assert len(_slow(TIMES, line)) > len(TIMES) // 10
 
 
 def test_items_by_their_number_alone_are_caught():
     by_number = [int(-(-t[1] // 16) * -(-t[0] // 32) >= 160) for t in SPLIT_TIMES]
     assert len(_slow(SPLIT_TIMES, by_number, 2)) > len(SPLIT_TIMES) // 10
+
+
+def test_rows_of_an_item(routes):
+    got = routes([t[:3] for t in ROW_TIMES])
+    assert [rows for _, _, rows in got] == [8 if t[3] < t[4] else 16 for t in ROW_TIMES]
