@@ -53,9 +53,10 @@
 // Workgroups are persistent over items; a workgroup's rounds form one stream
 // that runs on across its items.
 //
-// Matrices of 8,192 rows and more go to gemm_rows.hip up to 16 tokens, which
+// Matrices of 8,192 rows and more go to gemm_rows.hip at few tokens, which
 // cuts the work along rows (two or four waves per 16-row group for the whole
-// of K), and larger products of rows and tokens to gemm_tiles.hip.
+// of K), and larger products of rows and tokens to gemm_tiles.hip
+// (gemm_route.h).
 #include "gemm_route.h"
 #include "kernels.h"
 #include "q4_0_device.h"
@@ -504,16 +505,6 @@ hipError_t launch_tokens(const GemmParams &Pm, hipStream_t stream) {
 
 }  // namespace
 
-// From this many rows on, the row-split kernel up to 16 tokens and the
-// whole-prompt kernel (gemm_tiles.hip) past that: at 8192 x 2048 6.6 against
-// 8.3 us at 16 tokens, 9.3 against 8.3 at 17; gate|up 7.9 and 9.0 at 16, 10.2
-// and 9.5 at 24; the LM head 47 and 59 at 16, 80 and 51 at 17. (Its kernels
-// for 17 to 64 tokens, now gone, took 14.9 us at gate|up and 64 tokens against
-// 13.3.) At 3,072 rows the row-split kernel was twice as slow as this file's
-// (48 workgroups).
-constexpr int ROWS_MIN = 8192;
-constexpr int ROWS_MAX_M = 16;
-
 hipError_t launch_gemm(const MatrixRef &w, const uint8_t *x, int m, float *y, hipStream_t stream) {
     // One token is the M = 1 GEMV, byte for byte by the contract, and faster.
     // A few tokens are its weight stream with the arithmetic per token
@@ -537,11 +528,11 @@ hipError_t launch_gemm(const MatrixRef &w, const uint8_t *x, int m, float *y, hi
     if ((size_t)P.rows * (size_t)(P.k / QK * Q4_0_BYTES) >= 0x7fff0000u ||
         (size_t)64 * P.rows * 4 >= 0x7fff0000u)
         return hipErrorInvalidValue;
-    const bool by_rows = P.rows >= ROWS_MIN && gemm_rows_fits(P.rows, P.k);
-    if (by_rows ? m > ROWS_MAX_M : gemm_route::tiles_faster(m, P.rows, P.k, device_cu_count()))
-        return launch_gemm_tiles(P.w, x, m, y, P.rows, P.k, stream);
-    if (by_rows) return launch_gemm_rows(P.w, x, m, y, P.rows, P.k, stream);
-    return launch_tokens(P, stream);   // at most two covers of 32-token items: the outputs fit a range too
+    switch (gemm_route::form(m, P.rows, P.k, device_cu_count())) {
+        case gemm_route::ROWS: return launch_gemm_rows(P.w, x, m, y, P.rows, P.k, stream);
+        case gemm_route::TILES: return launch_gemm_tiles(P.w, x, m, y, P.rows, P.k, stream);
+        default: return launch_tokens(P, stream);   // at most two covers of 32-token items: the outputs fit a range too
+    }
 }
 
 }  // namespace w4a8

@@ -72,5 +72,26 @@ inline bool tiles_faster(int m, int rows, int k, int cus) {
     return k < (n16 == 3 && k % 1024 == 0 ? 2048 : 4096);
 }
 
+enum Form { SPLIT, ROWS, TILES };   // gemm_mfma.hip, gemm_rows.hip, gemm_tiles.hip
+
+// From ROWS_MIN rows on (and k a multiple of its 512-value segments) the
+// row-split kernel takes up to 16 tokens: at 8192 x 2048 6.6 us at 16 tokens
+// against 8.3 in the whole-prompt kernel, which has 8.3 against 9.3 at 17;
+// gate|up 7.9 and 9.0 at 16, 10.2 and 9.5 at 24; the LM head 47 and 59 at 16,
+// 80 and 51 at 17. (At 3,072 rows it was twice as slow as the class-split
+// kernel: 48 workgroups.) Up to 32 tokens it stays ahead on longer rows while
+// its workgroups of 64 rows are one cover of the CUs: 16384 x 8192 at 32
+// tokens 28.5 against 31.6, 8192 x 16384 50.4 against 55.9; at k = 2048 even,
+// and past one cover it loses (28672 x 8192 53.8 against 41.8).
+constexpr int ROWS_MIN = 8192;
+
+inline Form form(int m, int rows, int k, int cus) {
+    if (rows >= ROWS_MIN && k % 512 == 0) {
+        const bool two_tiles = m <= 32 && k >= 3072 && (rows + 63) / 64 <= cus;
+        return m <= 16 || two_tiles ? ROWS : TILES;
+    }
+    return tiles_faster(m, rows, k, cus) ? TILES : SPLIT;
+}
+
 }  // namespace gemm_route
 }  // namespace w4a8

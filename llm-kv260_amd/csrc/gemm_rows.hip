@@ -353,13 +353,13 @@ struct PairKernel {
 // accumulators 2q and 2q + 1, so it takes the blocks b with b % 8 in
 // {2q, 2q + 1}. At the end the tree's last adds, (p0 + p1) + (p2 + p3) with
 // p_q = a_2q + a_2q+1, meet through LDS: wave 0 of the group adds them.
-// PK = 2 (at most 8 tokens): packed tiles of two blocks.
-template <int GROUPS, int PK>
+// MT token tiles of 16 (two for 17 to 32 tokens). PK = 2 (at most 8 tokens):
+// packed tiles of two blocks.
+template <int MT, int GROUPS, int PK>
 struct QuadKernel {
-    static constexpr int MT = 1;             // token tiles of 16
     using G = Geo<MT, GROUPS, 4>;
     using S = Stager<G>;
-    static_assert(PK == 1 || PK == 2, "packed quads: two blocks of at most 8 tokens a tile");
+    static_assert(PK == 1 || (PK == 2 && MT == 1), "packed quads: two blocks of at most 8 tokens a tile");
 
     // Block B of the wave's view of the segment (the wave's blocks start at
     // 2q, folded into the pointers; B keeps the parity): its MFMA sums for
@@ -499,10 +499,9 @@ struct QuadKernel {
 
         // The tree: p_q = a_2q + a_2q+1 (PK = 2: across the lane halves),
         // then waves 1..3 hand their parts to wave 0.
-        constexpr int NT = PK == 2 ? 1 : MT;
-        float part[NT][4];
+        float part[MT][4];
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 part[t][r] = PK == 2 ? acc[0][0][r] + __shfl_xor(acc[0][0][r], 32) : acc[0][t][r] + acc[1][t][r];
@@ -513,7 +512,7 @@ struct QuadKernel {
         float *ex = reinterpret_cast<float *>(lds) + grp * 3 * G::TT * 16;
         if (q != 0 && holder) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+            for (int t = 0; t < MT; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) ex[((q - 1) * G::TT + 16 * t + tok0 + r) * 16 + j] = part[t][r];
         }
@@ -521,7 +520,7 @@ struct QuadKernel {
         if (q == 0) {
             const bool row_ok = holder && n0 + j < P.rows;
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+            for (int t = 0; t < MT; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int tok = 16 * t + tok0 + r;
@@ -539,10 +538,10 @@ __global__ __launch_bounds__(PairKernel::G::THREADS) void gemm_rows_pair_kernel(
     PairKernel::run(P, lds);
 }
 
-template <int GROUPS, int PK>
+template <int MT, int GROUPS, int PK>
 __global__ __launch_bounds__(64 * 4 * GROUPS) void gemm_rows_quad_kernel(RowsParams P) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    QuadKernel<GROUPS, PK>::run(P, lds);
+    QuadKernel<MT, GROUPS, PK>::run(P, lds);
 }
 
 template <class G>
@@ -554,9 +553,9 @@ hipError_t launch_rows(void (*kernel)(RowsParams), const RowsParams &P, hipStrea
     return hipGetLastError();
 }
 
-template <int GROUPS, int PK>
+template <int MT, int GROUPS, int PK>
 hipError_t launch_rows_quad(const RowsParams &P, hipStream_t stream) {
-    return launch_rows<typename QuadKernel<GROUPS, PK>::G>(&gemm_rows_quad_kernel<GROUPS, PK>, P, stream, GROUPS);
+    return launch_rows<typename QuadKernel<MT, GROUPS, PK>::G>(&gemm_rows_quad_kernel<MT, GROUPS, PK>, P, stream, GROUPS);
 }
 
 }  // namespace
@@ -565,9 +564,9 @@ bool gemm_rows_fits(int rows, int k) {
     return k % SEG == 0 && (size_t)rows * (size_t)(k / QK * Q4_0_BYTES) < 0x7fff0000u;
 }
 
-// m <= 16 tokens; y is [m][rows].
+// m <= 32 tokens; y is [m][rows].
 hipError_t launch_gemm_rows(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, hipStream_t stream) {
-    if (m < 1 || m > 16 || !gemm_rows_fits(rows, k)) return hipErrorInvalidValue;
+    if (m < 1 || m > 32 || !gemm_rows_fits(rows, k)) return hipErrorInvalidValue;
     RowsParams P{};
     P.w = w;
     P.x = x;
@@ -580,8 +579,9 @@ hipError_t launch_gemm_rows(const uint8_t *w, const uint8_t *x, int m, float *y,
     // One token tile: two 16-row groups a workgroup, two workgroups a CU
     // (four groups a workgroup were slower: gate|up at 8 / 16 tokens 8.8
     // against 8.3 / 8.4 us, the LM head 48.2 / 51.7 against 43.6 / 49.5).
-    if (m <= 8) return launch_rows_quad<2, 2>(P, stream);
-    return launch_rows_quad<2, 1>(P, stream);
+    if (m <= 8) return launch_rows_quad<1, 2, 2>(P, stream);
+    if (m <= 16) return launch_rows_quad<1, 2, 1>(P, stream);
+    return launch_rows_quad<2, 4, 1>(P, stream);   // four groups share two tiles' activations
 }
 
 }  // namespace w4a8

@@ -84,7 +84,7 @@ bool gemv_mt_fits(int m, int rows, int k);
 // The largest m for which it is the faster kernel on this shape.
 int gemv_mt_max_m(int rows, int k);
 hipError_t launch_gemv_mt(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, hipStream_t stream);
-// The row-split M > 1 kernel (gemm_rows.hip): m <= 16, k % 512 == 0.
+// The row-split M > 1 kernel (gemm_rows.hip): m <= 32, k % 512 == 0.
 bool gemm_rows_fits(int rows, int k);
 hipError_t launch_gemm_rows(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, hipStream_t stream);
 // Many tokens in one launch (gemm_tiles.hip): any m, rows and k whose weights fit a 32-bit byte count.

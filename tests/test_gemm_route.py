@@ -78,6 +78,14 @@ ROW_TIMES = (
     (16, 4096, 8192, 16.2, 10.7),
 )
 
+# m, rows, k, then microseconds: row-split and whole-prompt kernel, matrices of many rows.
+MANY_ROWS_TIMES = (
+    (16, 8192, 2048, 6.6, 8.3), (17, 8192, 2048, 9.3, 8.3), (24, 16384, 2048, 10.2, 9.5), (16, 128256, 2048, 47, 59),
+    (17, 128256, 2048, 80, 51), (32, 8192, 8192, 27.2, 29.1), (32, 9216, 4096, 15.7, 16.6), (28, 12288, 8192, 27.8, 29.4),
+    (17, 16384, 8192, 28.5, 30.5), (32, 16384, 4096, 16.6, 17.5), (32, 16384, 16384, 52.4, 59.0),
+    (32, 28672, 8192, 53.8, 41.8), (17, 28672, 4096, 30.3, 24.7), (33, 16384, 8192, 41.8, 39.3),
+)
+
 
 def _covers(m, rows, tokens):
     return -(-(-(-rows // 16) * -(-m // tokens)) // CUS)
@@ -98,10 +106,8 @@ def routes(tmp_path_factory):
     def run(sizes):
         text = "".join(f"{m} {rows} {k} {CUS}\n" for m, rows, k in sizes)
         out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=60).stdout
-        # Per size: the class-split kernel's items and the form taken, as indices into a
-        # row's times, and its rows per item.
-        return [(int(s == "split32"), 2 if f == "tiles" else int(s == "split32"), int(r[4:]))
-                for s, r, f in (line.split() for line in out.splitlines())]
+        # Per size: the class-split kernel's tokens and rows per item, and the form taken.
+        return [(int(t[5:]), int(r[4:]), f) for t, r, f in (line.split() for line in out.splitlines())]
     return run
 
 
@@ -110,20 +116,24 @@ def _slow(times, chosen, forms=3):
     return [(t[:3], c) for t, c in zip(times, chosen) if t[3 + c] > 1.06 * min(t[3:3 + forms])]
 
 
+def _index(tokens, form="split"):
+    return 2 if form == "tiles" else int(tokens == 32)
+
+
 def test_items_of_the_class_split_kernel(routes):
     got = routes([t[:3] for t in SPLIT_TIMES])
-    assert not _slow(SPLIT_TIMES, [split for split, _, _ in got], 2)
+    assert not _slow(SPLIT_TIMES, [_index(tokens) for tokens, _, _ in got], 2)
 
 
 def test_form_taken(routes):
     got = routes([t[:3] for t in TIMES])
-    assert not _slow(TIMES, [form for _, form, _ in got])
+    assert not _slow(TIMES, [_index(tokens, form) for tokens, _, form in got])
 
 
 def test_line_in_rows_times_tokens_is_caught(routes):
     got = routes([t[:3] for t in TIMES])
-    line = [2 if t[0] * t[1] >= (45000 if t[2] % 512 else 220000 - 42600000 // t[2]) else split
-            for t, (split, _, _) in zip(TIMES, got)]
+    line = [2 if t[0] * t[1] >= (45000 if t[2] % 512 else 220000 - 42600000 // t[2]) else _index(tokens)
+            for t, (tokens, _, _) in zip(TIMES, got)]
     assert len(_slow(TIMES, line)) > len(TIMES) // 10
 
 
@@ -134,4 +144,9 @@ def test_items_by_their_number_alone_are_caught():
 
 def test_rows_of_an_item(routes):
     got = routes([t[:3] for t in ROW_TIMES])
-    assert [rows for _, _, rows in got] == [8 if t[3] < t[4] else 16 for t in ROW_TIMES]
+    assert [rows for _, rows, _ in got] == [8 if t[3] < t[4] else 16 for t in ROW_TIMES]
+
+
+def test_many_rows(routes):
+    got = routes([t[:3] for t in MANY_ROWS_TIMES])
+    assert [form for _, _, form in got] == ["rows" if t[3] < t[4] else "tiles" for t in MANY_ROWS_TIMES]

@@ -298,7 +298,10 @@ def test_gemv_quarters_at_separate_addresses(gpu):
                                       # (8 | 9, 16 | 17, 32 | 33 tokens), ragged rows (not a whole
                                       # workgroup of 32 or 64), 1-4 K segments
                                       (9, 8200, 1024), (16, 8208, 2048), (17, 8200, 1536),
-                                      (32, 8200, 512), (33, 8240, 1024), (64, 8200, 2048)])
+                                      (32, 8200, 512), (33, 8240, 1024), (64, 8200, 2048),
+                                      # the row-split quads' two token tiles (17 to 32 tokens, K >= 3072):
+                                      # one token past a tile, both tiles full, ragged rows
+                                      (17, 8200, 3072), (32, 8208, 4096), (25, 8261, 3584)])
 def test_gemm_matches_rowwise_contract(gpu, m, rows, k):
     w = O.normal_f32((rows, k), 200 + m, 0.02)
     x = O.normal_f32((m, k), 300 + m)
