@@ -10,10 +10,15 @@
 //    F = MAGIC + 16 sumi (|16 sumi| <= 2^19, exact), and
 //    fma(F, d_w / 16, -MAGIC * d_w / 16) is sumi * d_w rounded once: F and
 //    the 13-bit product MAGIC * d_w / 16 are exact for every finite scale. An
-//    infinite or NaN scale gives NaN here, whatever the contract gives, and a
-//    NaN stays: an output that comes out NaN is computed again by the
-//    contract's own operations (plain_output) after it is stored. (A zero
-//    term's sign may differ; accumulators start at +0.0f and never see it.)
+//    infinite or NaN d_w gives NaN here, whatever the contract gives, and a
+//    NaN stays: a workgroup with an output that comes out NaN looks its rows'
+//    scales over, and if one is not finite runs its tile once more by the
+//    contract's own four operations: 2048 x 8192 at 512 tokens 40 us, 44 with
+//    every output NaN from the activations, 79 with a bad scale in every row
+//    (each NaN output by itself in one lane had taken 1,855). (With finite d_w the first product is the
+//    contract's, so a NaN from d_x is too. Only a zero's sign may differ: an
+//    accumulator starts at +0.0f and never sees it, and a NaN made of it and
+//    an infinite d_x has the same bits either way.)
 //  * A wave's tile is 64 rows x 64 tokens (64 x 32 where that leaves CUs
 //    idle), so that a block's weights are unpacked once for 64 tokens and
 //    each operand read from LDS meets four MFMAs.
@@ -98,46 +103,8 @@ struct TileGeo {
     static constexpr int D_LOADS = TT / 32;
     static constexpr int LOADS = 1 + X_LOADS;    // of every wave; one more in the first 1 + D_LOADS
     static_assert(X_OFF == 1024 * (WAVES + 1) && TT % (4 * WAVES) == 0, "the loads below");
-    static_assert(2 * LDS <= 160 * 1024, "two workgroups a CU");
+    static_assert(2 * (LDS + 1024) <= 160 * 1024, "two workgroups a CU, the vote's words among them");
 };
-
-// One output by the contract's operations as written (step 1's dot over the
-// block's bytes, convert, two multiplies, add; the tree by pairs).
-__device__ __forceinline__ float plain_output(const uint8_t *wrow, const uint8_t *xrow, int k) {
-    const float *xd = reinterpret_cast<const float *>(xrow + k);
-    float quad = 0.0f, half = 0.0f, sum = 0.0f;
-#pragma unroll 1
-    for (int p = 0; p < 4; ++p) {
-        float l[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            float acc = 0.0f;
-#pragma unroll 1
-            for (int b = 2 * p + e; b < k / QK; b += 8) {
-                const uint16_t *blk = reinterpret_cast<const uint16_t *>(wrow + (size_t)b * Q4_0_BYTES);
-                const uint32_t *xb = reinterpret_cast<const uint32_t *>(xrow + QK * b);
-                uint32_t qs[4], lo[4], hi[4], xr[8];
-                int32_t sum_x = 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) qs[i] = (uint32_t)blk[1 + 2 * i] | ((uint32_t)blk[2 + 2 * i] << 16);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    xr[i] = xb[i];
-                    sum_x = __builtin_amdgcn_sdot4((int)xr[i], 0x01010101, sum_x, false);
-                }
-                unpack_nibbles(qs, lo, hi);
-                acc = acc + block_term(block_dot_raw(lo, hi, xr, -8 * sum_x), blk[0], xd[b]);
-            }
-            l[e] = acc;
-        }
-        const float pair = l[0] + l[1];
-        if (p == 0) quad = pair;
-        if (p == 1) quad = quad + pair;
-        if (p == 2) half = pair;
-        if (p == 3) sum = quad + (half + pair);
-    }
-    return sum;
-}
 
 template <int NT>
 struct TileKernel {
@@ -148,8 +115,7 @@ struct TileKernel {
         uint32_t w, x[G::X_LOADS], p;
         int p_lds;                        // the last load's offset in a buffer, -1 for none
     };
-    static __device__ __forceinline__ void slots(const TileParams &P, int row_bytes, int w, Slots &s) {
-        const int lane = threadIdx.x & 63;
+    static __device__ __forceinline__ void slots(const TileParams &P, int row_bytes, int w, int lane, Slots &s) {
         auto w_piece = [&](int q) {
             const int r = q / CHUNK_PIECES, p = q - CHUNK_PIECES * r;
             return (uint32_t)r * (uint32_t)row_bytes + 16u * (uint32_t)p;
@@ -233,8 +199,7 @@ struct TileKernel {
         int nib, scl, xa, dx;
         uint32_t shift;
     };
-    static __device__ __forceinline__ Lane lane_offsets(int b) {
-        const int lane = threadIdx.x & 63;
+    static __device__ __forceinline__ Lane lane_offsets(int b, int lane) {
         const int j = lane & 15, g = lane >> 4, up = g >> 1, odd = b & 1;
         Lane L;
         L.scl = j * G::WP + 18 * b;
@@ -245,8 +210,11 @@ struct TileKernel {
         return L;
     }
 
-    // One block's terms, added to the wave's accumulator.
-    static __device__ __forceinline__ void block(const uint8_t *buf, const Lane &L, const v4i &magic, float acc[NT][RT][4]) {
+    // One block's terms, added to the wave's accumulator; PLAIN by the
+    // contract's operations as written. `bias` is what the MFMAs add their
+    // sums to: MAGIC's bits, or 0 if PLAIN.
+    template <bool PLAIN>
+    static __device__ __forceinline__ void block(const uint8_t *buf, const Lane &L, const v4i &bias, float acc[NT][RT][4]) {
         long wb[RT];
         float dw[RT], dm[RT];
 #pragma unroll
@@ -268,12 +236,12 @@ struct TileKernel {
             for (int e = 0; e < 4; ++e) dx[e] = *reinterpret_cast<const float *>(buf + L.dx + (16 * t + 4 * e) * 32);
             v4i d[RT];
 #pragma unroll
-            for (int r = 0; r < RT; ++r) d[r] = __builtin_amdgcn_mfma_i32_16x16x32_i8(ax, wb[r], magic, 0, 0, 0);
+            for (int r = 0; r < RT; ++r) d[r] = __builtin_amdgcn_mfma_i32_16x16x32_i8(ax, wb[r], bias, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < RT; ++r)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float a = __builtin_fmaf(__int_as_float(d[r][e]), dw[r], dm[r]);
+                    const float a = PLAIN ? (float)d[r][e] * dw[r] : __builtin_fmaf(__int_as_float(d[r][e]), dw[r], dm[r]);
                     acc[t][r][e] = acc[t][r][e] + a * dx[e];
                 }
         }
@@ -281,9 +249,8 @@ struct TileKernel {
 
     // Exchange of token tiles 2 h and 2 h + 1: the tree over the eight
     // accumulators, and the stores.
-    static __device__ __forceinline__ bool reduce_half(const TileParams &P, int n0, int m0, uint8_t *ex, int w, int h,
+    static __device__ __forceinline__ bool reduce_half(const TileParams &P, int n0, int m0, uint8_t *ex, int w, int lane, int h,
                                                        const float acc[NT][RT][4]) {
-        const int lane = threadIdx.x & 63;
         const int j = lane & 15, g = lane >> 4;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -315,20 +282,25 @@ struct TileKernel {
     }
 
     // The item at rows n0 .., tokens m0 ..: chunk c is computed from LDS
-    // buffer c % 2 while the loads of chunk c + 1 fill the other.
-    static __device__ __forceinline__ void run(const TileParams &P, int n0, int m0, uint8_t *lds) {
+    // buffer c % 2 while the loads of chunk c + 1 fill the other. Whether an
+    // output of this thread came out NaN.
+    template <bool PLAIN>
+    static __device__ __forceinline__ bool pass(const TileParams &P, int n0, int m0, uint8_t *lds) {
         const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        int lane = threadIdx.x & 63;
+        if constexpr (PLAIN) __asm__ volatile("" : "+v"(lane));   // else the first pass's offsets are kept for this one, and spill
         const int row_bytes = P.k / QK * Q4_0_BYTES;
         const int chunks = P.k / 256;
         const int base = (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
         Slots s;
-        slots(P, row_bytes, w, s);
+        slots(P, row_bytes, w, lane, s);
         Source S;
         source(P, row_bytes, n0, m0, w, S);
         load(s, S, w, base);
-        const Lane L = lane_offsets(w);
-        v4i magic = {MAGIC_BITS, MAGIC_BITS, MAGIC_BITS, MAGIC_BITS};
-        __asm__ volatile("" : "+v"(magic));
+        const Lane L = lane_offsets(w, lane);
+        constexpr int BIAS = PLAIN ? 0 : MAGIC_BITS;
+        v4i bias = {BIAS, BIAS, BIAS, BIAS};
+        __asm__ volatile("" : "+v"(bias));
         float acc[NT][RT][4];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
@@ -339,11 +311,11 @@ struct TileKernel {
         arrive();
         for (int c = 0;; c += RING) {
             if (c + 1 < chunks) load(s, S, w, base + G::BUF);   // last read for chunk c - 1, before the last barrier
-            block(lds, L, magic, acc);
+            block<PLAIN>(lds, L, bias, acc);
             arrive();
             if (c + 1 >= chunks) break;
             if (c + 2 < chunks) load(s, S, w, base);
-            block(lds + G::BUF, L, magic, acc);
+            block<PLAIN>(lds + G::BUF, L, bias, acc);
             arrive();
             if (c + 2 >= chunks) break;
         }
@@ -351,21 +323,30 @@ struct TileKernel {
 #pragma unroll
         for (int h = 0; h < NT / 2; ++h) {
             if (h) __syncthreads();                              // the half before is read
-            nan = reduce_half(P, n0, m0, lds, w, h, acc) || nan;
+            nan = reduce_half(P, n0, m0, lds, w, lane, h, acc) || nan;
         }
-        // Outputs that came out NaN, again and as the contract writes them.
-        if (nan) {
-            const int row = n0 + (int)(threadIdx.x & 63);
-#pragma unroll 1
-            for (int i = 0; i < 2 * NT; ++i) {
-                const int tok = m0 + 32 * (i >> 2) + 4 * w + (i & 3);
-                if (tok >= P.m) continue;
-                float *y = P.y + (size_t)tok * P.rows + row;
-                if (*y != *y) *y = plain_output(P.w + (size_t)row * row_bytes, P.x + (size_t)tok * P.x_stride, P.k);
-            }
-        }
+        return nan;
+    }
+
+    // Whether one of the blocks this thread looks at (a row's b, b + 8, ..) has a scale that is not finite.
+    static __device__ __forceinline__ bool scale_not_finite(const TileParams &P, int n0) {
+        const int row = n0 + ((int)threadIdx.x >> 3), nb = P.k / QK;
+        if (row >= P.rows) return false;
+        const uint8_t *src = P.w + (size_t)row * ((size_t)nb * Q4_0_BYTES);
+        bool bad = false;
+#pragma unroll 8
+        for (int b = threadIdx.x & 7; b < nb; b += 8)
+            bad |= (*reinterpret_cast<const uint16_t *>(src + (size_t)b * Q4_0_BYTES) & 0x7C00u) == 0x7C00u;
+        return bad;
+    }
+
+    static __device__ __forceinline__ void run(const TileParams &P, int n0, int m0, uint8_t *lds) {
+        // (the votes' barriers keep the exchange until every wave has read it)
+        if (!__syncthreads_or(pass<false>(P, n0, m0, lds))) return;
+        if (__syncthreads_or(scale_not_finite(P, n0))) pass<true>(P, n0, m0, lds);
     }
 };
+static_assert(THREADS == 8 * TILE_ROWS, "scale_not_finite: eight threads a row");
 
 template <int NT>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_tiles_kernel(TileParams P) {

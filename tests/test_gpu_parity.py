@@ -363,6 +363,66 @@ def test_gemm_whole_prompt(gpu, m, rows, k):
     assert (got[m].view(np.uint8) == 0xAA).all(), "written past the last token"
 
 
+@pytest.mark.parametrize("m,rows,k", [(70, 2100, 2304), (200, 3333, 2048)])   # 32- and 64-token tiles
+def test_gemm_whole_prompt_nonfinite_activations(gpu, m, rows, k):
+    """Activation scales that are not finite, weight scales that are: the NaN bits of
+    every kind, from sums of zero under either sign of the weight's scale too."""
+    rng = np.random.default_rng(413)
+    blocks = C.quantize_q4_0(O.normal_f32((rows, k), 414, 0.02)).reshape(rows, k // 32, 18)
+    blocks[::3, ::5, 2:] = 0x88                                                 # all weights 8 - 8 = 0
+    d = (rng.standard_normal((rows, k // 32)) * 0.01).astype(np.float16)        # either sign
+    blocks[..., :2] = d.view(np.uint8).reshape(rows, k // 32, 2)
+    blocks = blocks.reshape(rows, -1)
+    xq, xd = C.quantize_q8_0_rows(O.normal_f32((m, k), 415))
+    xd = xd.copy()
+    odd = np.array([0x7C00, 0xFC00, 0x7E00, 0xFE00, 0x7D01, 0xFD55], np.uint16).view(np.float16)   # inf, NaN of each kind
+    for t in range(0, m, 2):
+        b = 5 * rng.integers(0, k // 160)
+        xd[t, b] = odd[(t // 2) % 6]
+        if t % 8 == 0:   # a second one in another accumulator (which of two NaNs an add keeps is not the contract's)
+            xd[t, (b + rng.integers(1, 8)) % (k // 32)] = odd[(t // 8) % 6]
+    want = C.gemm_q4_0_rows(blocks, k, xq, xd)
+    assert np.isnan(want).any() and np.isinf(want).any()
+    x_rows = np.stack([C.pack_x_for_engine(xq[i], xd[i]) for i in range(m)])
+    y = poisoned_f32((m, rows))
+    gpu.gemm_engine(dev(blocks), k, dev(x_rows), out=y)
+    assert_bytes_equal(host(y), want, f"gemm {m}x{rows}x{k}, NaN bytes included")
+
+
+def test_gemm_whole_prompt_nonfinite_time(gpu):
+    """A prompt that comes out NaN takes at most four times a finite one's time (a tile is
+    looked over and run once more, not each output by itself): measured 1.1 times for NaN
+    activations, 2.2 for a weight scale that is not finite in every row."""
+    import torch
+    m, rows, k = 512, 2048, 8192
+    blocks = C.quantize_q4_0(O.normal_f32((64, k), 416, 0.02)).reshape(64, k // 32, 18)
+    bad = blocks.copy()
+    bad[:, 7, :2] = np.array([np.nan], np.float16).view(np.uint8)
+    w, w_bad = (dev(np.tile(b.reshape(64, -1), (rows // 64, 1))) for b in (blocks, bad))
+    x = gpu.quantize_q8_0_engine(dev(O.normal_f32((m, k), 417)))
+    x_bad = x.clone()
+    x_bad[:, k:].view(torch.float32)[:, 3] = float("nan")
+    y = torch.empty((m, rows), device="cuda")
+
+    def time(w, x):
+        best = float("inf")
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(5):
+                gpu.gemm_engine(w, k, x, out=y)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+
+    finite = time(w, x)
+    assert torch.isfinite(y).all()
+    for name, t in (("activations", time(w, x_bad)), ("weights", time(w_bad, x))):
+        assert torch.isnan(y).all()
+        assert t < 4 * finite, f"{name}: {t / finite:.1f} times a finite prompt's time"
+
+
 def test_gemm_one_row_equals_gemv(gpu):
     rows, k = 96, 2048
     _, _, blocks, xq, xd = _case(rows, k, 130, 131)
