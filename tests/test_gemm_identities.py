@@ -1,4 +1,4 @@
-"""The two identities the M > 1 MFMA kernels rest on, checked exhaustively on the CPU
+"""The identities the M > 1 MFMA kernels rest on, checked exhaustively on the CPU
 (the GPU parity tests run the kernels themselves against the oracle).
 
 - The weight operand (csrc/gemm_rows.hip block_weights, csrc/gemm_mfma.hip): each nibble
@@ -9,6 +9,10 @@
   equals the contract's f32(sumi) * d_w bit for bit, for every fp16 scale (subnormal,
   infinite and NaN included) and every block sum a block can have (|sumi| <= 32 * 8 *
   128). The same check with a factor that is not a power of two fails.
+- The biased sum (csrc/gemm_tiles.hip): the MFMA's 16 sumi added to the bits of
+  1.5 * 2^23 read as the float MAGIC + 16 sumi, and fma(MAGIC + 16 sumi, d_w / 16,
+  -MAGIC * (d_w / 16)) is the same product for every finite fp16 scale, but for the sign
+  of a zero, and NaN for every other. A bias too small for the sums fails.
 """
 import numpy as np
 
@@ -82,3 +86,37 @@ def test_scaled_product_check_catches_a_wrong_scaling():
     want = (np.float32(s) * d)[fin]
     wrong = (np.float32(3 * s) * (d / np.float32(3)))[fin]
     assert not np.array_equal(wrong.view(np.uint32), want.view(np.uint32))
+
+
+def _biased_product(s, d, magic):
+    """fma(float from bits(magic) + 16 s, d / 16, -magic * (d / 16)) in float32: the float64
+    value of a finite one is exact (24 + 11 bits, less a 13-bit product), so rounding it is
+    the fma's one rounding."""
+    f = (np.float32(magic).view(np.int32) + 16 * np.asarray(s, np.int32)).astype(np.int32).view(np.float32)
+    d16 = d * np.float32(0.0625)
+    dm = d16 * np.float32(-magic)
+    return (f.astype(np.float64) * d16.astype(np.float64) + dm.astype(np.float64)).astype(np.float32)
+
+
+@np.errstate(invalid="ignore", over="ignore")
+def test_biased_fma_equals_contract_product_for_every_fp16_scale():
+    d = np.arange(1 << 16, dtype=np.uint32).astype(np.uint16).view(np.float16).astype(np.float32)
+    fin = np.isfinite(d)
+    magic = 1.5 * 2.0 ** 23
+    exact = (d[fin] * np.float32(0.0625)).astype(np.float64) * magic
+    assert np.array_equal((d[fin] * np.float32(0.0625) * np.float32(magic)).astype(np.float64), exact)
+    every = np.arange(-32768, 32769)
+    for s, scales in [(np.int64(v), d) for v in (0, 1, -1, 2, -3, 300, 4095, -4097, 12345, -23456, 32767, 32768, -32768)] + \
+            [(every, d[i]) for i in (0x0001, 0x03FF, 0x0400, 0x2E66, 0xA123, 0x3C00, 0x7BFF, 0xFBFF)]:
+        ok = np.isfinite(scales)
+        got = _biased_product(s, scales, magic)
+        want = s.astype(np.float32) * scales
+        assert np.array_equal((got + np.float32(0))[ok].view(np.uint32), (want + np.float32(0))[ok].view(np.uint32))
+        assert np.isnan(got[~ok]).all()
+
+
+@np.errstate(invalid="ignore", over="ignore")
+def test_biased_fma_check_catches_a_small_bias():
+    d = np.float32(0.015625)
+    s = np.arange(-32768, 32769)
+    assert not np.array_equal(_biased_product(s, d, 1.5 * 2.0 ** 18), s.astype(np.float32) * d)

@@ -268,12 +268,12 @@ def test_gemv_quarters_at_separate_addresses(gpu):
                                       # one chunk per row; three and five chunks (rounds of one chunk);
                                       # several 64-token groups; one row
                                       (8, 16, 256), (40, 33, 768), (130, 40, 1280), (2, 1, 512),
-                                      # 8192 rows and more go to the row-split kernel: ragged row
-                                      # groups and workgroups, one to three token tiles, several
-                                      # 64-token groups, one to four K segments
+                                      # 8192 rows and more: the row-split kernel at few tokens, the
+                                      # whole-prompt kernel past 16 (short rows); ragged row groups and
+                                      # workgroups, several 64-token groups, one to four K segments
                                       (3, 8200, 512), (17, 8208, 1024), (40, 8240, 2048), (64, 8192, 512),
                                       (130, 8256, 1536),
-                                      # the largest K, on both kernels
+                                      # the largest K, class-split and row-split
                                       (40, 64, 16384), (5, 8200, 16384),
                                       # the few-token GEMV (m = 2, or m <= 4 on large matrices, m <= 6
                                       # where they have at most four tiles per CU and a tile's tokens
@@ -291,11 +291,12 @@ def test_gemv_quarters_at_separate_addresses(gpu):
                                       (33, 1001, 8192),
                                       # the row-split kernel's packed tiles: 2 blocks x 8 tokens (m = 5..8)
                                       # and 4 blocks x 4 tokens (m <= 4 where the few-token GEMV does not
-                                      # take the shape); ragged rows, 1-3 K segments
+                                      # take the shape); ragged rows, 1-3 K segments (69 tokens: the
+                                      # whole-prompt kernel)
                                       (5, 8200, 2048), (8, 8256, 4096), (7, 9000, 1536), (6, 8192, 512),
                                       (4, 8200, 12288), (2, 8193, 1024), (69, 8200, 1024),
-                                      # the row-split quads on each side of their token tilings
-                                      # (8 | 9, 16 | 17, 32 | 33 tokens), ragged rows (not a whole
+                                      # the row-split quads past 8 tokens, and from 17 on these short
+                                      # rows in the whole-prompt kernel; ragged rows (not a whole
                                       # workgroup of 32 or 64), 1-4 K segments
                                       (9, 8200, 1024), (16, 8208, 2048), (17, 8200, 1536),
                                       (32, 8200, 512), (33, 8240, 1024), (64, 8200, 2048),
@@ -315,10 +316,12 @@ def test_gemm_matches_rowwise_contract(gpu, m, rows, k):
 
 
 @pytest.mark.parametrize("m,rows,k", [(24, 8200, 1024), (40, 2000, 1024), (2, 2000, 2048), (4, 8200, 2048),
-                                      (3, 600, 8192), (9, 1003, 8192), (7, 8200, 2048), (3, 8200, 512)])
+                                      (3, 600, 8192), (9, 1003, 8192), (7, 8200, 2048), (3, 8200, 512),
+                                      (20, 8200, 3072), (300, 2000, 768)])
 def test_gemm_random_bytes(gpu, m, rows, k):
-    """Arbitrary block bytes and activations (any finite fp16 scale) through both M > 1
-    kernels (8,200 rows: the row-split one), row by row against the contract."""
+    """Arbitrary block bytes and activations (any finite fp16 scale) through every M > 1
+    kernel (24 tokens of 8,200 rows and 300 of 2,000 are the whole-prompt one's, in tiles of
+    32 and 64 tokens), row by row against the contract."""
     rng = np.random.default_rng(78 + m)
     blocks = rng.integers(0, 256, size=(rows, k // 32, 18), dtype=np.uint8)
     d = (rng.standard_normal((rows, k // 32)) * 10.0 ** rng.integers(-7, 3, (rows, k // 32))).astype(np.float16)
@@ -335,7 +338,7 @@ def test_gemm_random_bytes(gpu, m, rows, k):
 
 @pytest.mark.parametrize("m,rows,k", [
     (65, 700, 256), (1100, 128, 256),       # one chunk; many 32-token groups of few rows
-    (33, 1400, 768), (129, 1601, 768),      # odd chunk counts, a last group of one token, of one row
+    (33, 1400, 768), (33, 2100, 768), (129, 1601, 768),      # odd chunk counts, a last group of one token, of one row
     (96, 2305, 512), (97, 2309, 1024),      # whole 32-token groups, one token more
     (17, 8200, 512), (6, 8300, 768),        # many rows, few tokens
     (40, 8200, 512), (70, 8200, 256),       # 64-token tiles: 40 of 64, a last group of 6
@@ -361,6 +364,25 @@ def test_gemm_whole_prompt(gpu, m, rows, k):
     got = host(y)
     assert_bytes_equal(got[:m], want, f"gemm {m}x{rows}x{k}")
     assert (got[m].view(np.uint8) == 0xAA).all(), "written past the last token"
+
+
+@pytest.mark.parametrize("m,rows,k", [(150, 3400, 8192),    # 64-token tiles, 32 chunks, a last group of 22 tokens
+                                      (333, 3333, 2304),    # 64-token tiles, 9 chunks, ragged rows
+                                      (40, 4200, 16128),    # 32-token tiles, 63 chunks
+                                      (200, 1800, 16384)])  # the longest rows
+def test_gemm_whole_prompt_long_rows(gpu, m, rows, k):
+    blocks = C.quantize_q4_0(O.normal_f32((rows, k), 411, 0.02)).reshape(rows, k // 32, 18)
+    blocks[rows - 70, -2, :2] = np.array([np.inf], np.float16).view(np.uint8)    # in the last chunk, a tile of its own
+    blocks[5, k // 64, :2] = np.array([-np.inf], np.float16).view(np.uint8)
+    blocks = blocks.reshape(rows, -1)
+    xq, xd = C.quantize_q8_0_rows(O.normal_f32((m, k), 412))
+    xq = xq.copy()
+    xq[m - 1, -32:] = -128
+    want = C.gemm_q4_0_rows(blocks, k, xq, xd)
+    x_rows = np.stack([C.pack_x_for_engine(xq[i], xd[i]) for i in range(m)])
+    y = poisoned_f32((m, rows))
+    gpu.gemm_engine(dev(blocks), k, dev(x_rows), out=y)
+    assert_bytes_equal(host(y), want, f"gemm {m}x{rows}x{k}")
 
 
 @pytest.mark.parametrize("m,rows,k", [(70, 2100, 2304), (200, 3333, 2048)])   # 32- and 64-token tiles
