@@ -21,13 +21,16 @@
 // sequence holding their 64 best, which six compare-exchange steps sort.
 //
 // Stage 2: one workgroup, so all of it is latency (a chain of shuffles,
-// barriers and loads), and it sorts as little as it can. With at least k
-// lists, the k-th largest list head is a bound no larger than the k-th best
-// key: the heads are sorted first (two to four lists of 64), the keys at or
-// above the bound gathered (about k of them for random logits), and up to 256
-// of them sorted and merged. More, or fewer lists than k, take the merge of
-// all lists pairwise, level by level. 128,256 logits, a call of both stages:
-// 14.4 us with the pairwise merge and shuffles through LDS, 12.5 so.
+// barriers and loads). Up to 64 lists it merges them pairwise, level by level.
+// Past that it sorts as little as it can: the k-th largest list head is a
+// bound no larger than the k-th best key, so the heads are sorted first, the
+// keys at or above the bound gathered (about k of them for random logits), and
+// up to 256 of them sorted and merged. More (ties, or candidates close
+// together) are in exactly the k lists whose heads reach the bound, and only
+// these are merged. A call of both stages, k = 40, MI355X: 128,256 logits 12.2
+// us (14.0 with all lists merged pairwise), tied 14.6 (14.1); 262,144 12.4 (17.1) and
+// 14.9; 16,000 and 64,000, merged pairwise, 10.5 and 11.9 (12.2 and 12.9 by
+// heads); one list 8.8 (11.8).
 //
 // A NaN logit has no place in that order: the reference's loop admits it
 // (v <= NaN is false) into the last slot, evicting the k-th candidate it
@@ -49,7 +52,8 @@ namespace {
 
 constexpr int TOPK_SLICE = 1024;      // logits per stage-1 workgroup
 constexpr int TOPK_LIST = 64;         // candidates each list keeps (k <= 64)
-constexpr int TOPK_MAX_LISTS = 256;   // stage 2's LDS: 256 x 64 keys = 128 KB
+constexpr int TOPK_MAX_LISTS = 256;
+constexpr int TOPK_MERGE_LISTS = 64;  // lists stage 2 merges pairwise, 32 KB of LDS (k <= 64 of them past this many)
 constexpr int TOPK_CAND = 256;        // keys stage 2 sorts without the pairwise merge (and list heads)
 static_assert(TOPK_LIST == 64 && TOPK_CAND == 4 * TOPK_LIST && TOPK_CAND >= TOPK_MAX_LISTS,
               "the index arithmetic below takes lists of 64, four of them in `cand`");
@@ -219,10 +223,11 @@ __global__ __launch_bounds__(1024) void topk_stage2(const float *__restrict__ y,
                                                     const unsigned long long *lists, int nlists, int k,
                                                     float *__restrict__ vals,
                                                     int32_t *__restrict__ idx) {
-    extern __shared__ __attribute__((aligned(16))) unsigned long long lk[];
+    __shared__ __attribute__((aligned(16))) unsigned long long lk[TOPK_MERGE_LISTS * TOPK_LIST];
     __shared__ unsigned long long cand[TOPK_CAND];
-    __shared__ int n_cand;
+    __shared__ int n_cand, n_merge;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const bool by_heads = nlists > TOPK_MERGE_LISTS;
     // Up to 16 keys per thread (256 lists of 64), all loaded before any is
     // used: key j is place `lane` of list 16 j + wave; missing lists are empty
     // (key 0).
@@ -236,8 +241,8 @@ __global__ __launch_bounds__(1024) void topk_stage2(const float *__restrict__ y,
         kv[j] = lists[i < have ? i : have - 1];
     }
     // Four waves sort the heads, 64 each.
-    if (t < TOPK_CAND) cand[t] = sort64(t < nlists ? head : 0ull, lane);
-    if (t == 0) n_cand = 0;
+    if (by_heads && t < TOPK_CAND) cand[t] = sort64(t < nlists ? head : 0ull, lane);
+    if (t == 0) n_cand = n_merge = 0;
     if (__syncthreads_or(t < nlists && head == NAN_MARK)) {
         if (wave == 0) topk_in_order(y, n, k, vals, idx, lane);
         return;
@@ -251,12 +256,12 @@ __global__ __launch_bounds__(1024) void topk_stage2(const float *__restrict__ y,
         const unsigned long long b = merge64(cand[128 + lane], cand[255 - lane], lane);
         return merge64(a, reversed(b, lane), lane);
     };
-    bool done = false;
+    int merge_lists = nlists;                     // lists to merge pairwise, in lk
     unsigned long long out = 0ull;
-    if (nlists >= k) {
+    if (by_heads) {
         const unsigned long long heads = best_of_four();
-        // The k-th largest head (k <= nlists: it is a list's, and 0 only if
-        // that list is empty). Keys differ, so k keys at least reach it.
+        // The k-th largest head (k <= 64 < nlists: it is a list's, and 0 only
+        // if that list is empty). Keys differ, so k keys at least reach it.
         const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)heads, k - 1);
         const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(heads >> 32), k - 1);
         const unsigned long long bound = max_u64(((unsigned long long)hi << 32) | lo, 1ull);
@@ -269,8 +274,8 @@ __global__ __launch_bounds__(1024) void topk_stage2(const float *__restrict__ y,
         at = __builtin_amdgcn_readfirstlane(at);
         __syncthreads();                          // the heads are read in every wave, the count is whole
         const int total = n_cand;
-        done = total <= TOPK_CAND;
-        if (done) {
+        if (total <= TOPK_CAND) {
+            merge_lists = 0;
 #pragma unroll
             for (int j = 0; j < KEYS; ++j) {
                 const unsigned long long m = __ballot(kv[j] >= bound);
@@ -288,15 +293,29 @@ __global__ __launch_bounds__(1024) void topk_stage2(const float *__restrict__ y,
                 __syncthreads();
                 if (wave == 0) out = best_of_four();
             }
-        }
-    }
-    if (!done) {
-        int np = 1;
-        while (np < nlists) np <<= 1;
+        } else {
+            // The lists whose head reaches the bound, at most k. (Counted here
+            // and not with the keys: there it cost every call 0.4 us.)
+            int mine = 0, slot = 0;
 #pragma unroll
-        for (int j = 0; j < KEYS; ++j) {
-            const int i = t + 1024 * j;
-            if (i < np * TOPK_LIST) lk[i] = kv[j];
+            for (int j = 0; j < KEYS; ++j) mine += __ballot(kv[j] >= bound) != 0;
+            if (lane == 0) slot = atomicAdd(&n_merge, mine);
+            slot = __builtin_amdgcn_readfirstlane(slot);
+#pragma unroll
+            for (int j = 0; j < KEYS; ++j)
+                if (__ballot(kv[j] >= bound)) lk[(slot++) * TOPK_LIST + lane] = kv[j];
+            __syncthreads();
+            merge_lists = n_merge;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < TOPK_MERGE_LISTS / 16; ++j) lk[t + 1024 * j] = kv[j];
+    }
+    if (merge_lists) {
+        int np = 1;
+        while (np < merge_lists) np <<= 1;
+        if (by_heads) {                           // empty lists up to a power of two
+            for (int i = merge_lists * TOPK_LIST + t; i < np * TOPK_LIST; i += 1024) lk[i] = 0ull;
         }
         // Level by level: lists a = 2 g s and b = a + s meet into a, a wave per pair.
         for (int s = 1; s < np; s <<= 1) {
@@ -381,15 +400,10 @@ hipError_t launch_topk(const float *y, int n, int k, float *vals, int32_t *idx, 
     const int nlists = (n + TOPK_SLICE - 1) / TOPK_SLICE;
     if (n < 1 || nlists > TOPK_MAX_LISTS || k < 1 || k > TOPK_LIST) return hipErrorInvalidValue;
     auto *lists = static_cast<unsigned long long *>(workspace);
-    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void *>(&topk_stage2), 160 * 1024);
-    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(topk_stage1, dim3((unsigned)nlists), dim3(256), 0, stream, y, n, lists);
-    e = hipGetLastError();
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    int np = 1;
-    while (np < nlists) np <<= 1;
-    const size_t lds = (size_t)np * TOPK_LIST * sizeof(unsigned long long);
-    hipLaunchKernelGGL(topk_stage2, dim3(1), dim3(1024), lds, stream, y, n, lists, nlists, k, vals, idx);
+    hipLaunchKernelGGL(topk_stage2, dim3(1), dim3(1024), 0, stream, y, n, lists, nlists, k, vals, idx);
     return hipGetLastError();
 }
 

@@ -59,11 +59,14 @@ def test_special_values(gpu):
     _check(gpu, np.zeros(4096, dtype=np.float32), 64, "all zero")
 
 
-@pytest.mark.parametrize("n,k", [(65536, 64), (65536 - 1024, 64), (8192, 8), (8192, 9), (262144, 64), (262143, 40)])
-@pytest.mark.parametrize("how", ["one slice", "few slices", "every slice", "descending", "negative zeros"])
+@pytest.mark.parametrize("n,k", [(65536, 64), (65536 - 1024, 64), (65537, 64), (66561, 1), (128256, 40), (8192, 8),
+                                 (8192, 9), (1025, 2), (1024, 1), (262144, 64), (262143, 40)])
+@pytest.mark.parametrize("how", ["one slice", "few slices", "every slice", "descending", "negative zeros",
+                                 "few admitted", "six slices admitted"])
 def test_topk_where_the_best_lie(gpu, n, k, how):
-    """Lists (1,024 logits each) as many as k and one fewer or more, and candidates at or above
-    the k-th list head from one list's 64 up to more than the 256 that are sorted by themselves."""
+    """Lists (1,024 logits each) as many as are merged pairwise (64), one more, one, and k;
+    candidates at or above the k-th list head from one list's 64 up to more than the 256 that
+    are sorted by themselves."""
     y = _logits(n, n + k)
     rng = np.random.default_rng(k)
     if how == "one slice":
@@ -74,6 +77,10 @@ def test_topk_where_the_best_lie(gpu, n, k, how):
     elif how == "every slice":              # each slice a full list above the rest
         for c in range(n // 1024):
             y[1024 * c + 100:1024 * c + 164] += 50.0
+    elif how == "few admitted":             # fewer lists with a candidate than k, mostly
+        y = np.where(np.arange(n) % (n // 5) == 0, y, F32(-1e30))
+    elif how == "six slices admitted":      # as few lists, and more than 256 candidates
+        y = np.where(np.arange(n) // 1024 % max(n // 6144, 1) == 0, y, F32(-1e30))
     elif how == "descending":
         y = np.sort(y)[::-1].copy()
     else:                                   # ties of +0 and -0, their bits kept
@@ -81,6 +88,38 @@ def test_topk_where_the_best_lie(gpu, n, k, how):
         at = rng.choice(n, 200, replace=False)
         y[at] = np.where(np.arange(200) % 2, F32(0.0), F32(-0.0))
     _check(gpu, y, k, f"n={n} k={k} {how}")
+
+
+def test_topk_time_where_the_bound_does_not_help(gpu):
+    """A call of one list has nothing to sort by heads, and where hundreds of candidates tie
+    only the lists that hold them are merged: measured 0.72 times a call of 128,256 logits, and
+    1.15 times the same call on random logits."""
+    import torch
+
+    def time(y, k):
+        y = dev(y)
+        ws = torch.empty(gpu.lib().w4a8_topk_workspace_bytes(y.numel()), dtype=torch.uint8, device="cuda")
+        vals, idx = torch.empty(k, device="cuda"), torch.empty(k, dtype=torch.int32, device="cuda")
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            s = torch.cuda.current_stream().cuda_stream
+            for _ in range(40):
+                gpu.check("w4a8_topk", gpu.lib().w4a8_topk(y.data_ptr(), y.numel(), k, vals.data_ptr(), idx.data_ptr(),
+                                                           ws.data_ptr(), ws.numel(), s))
+        best = float("inf")
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            g.replay()
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+
+    small, large = time(_logits(1000, 1), 1), time(_logits(128256, 2), 40)
+    assert small < 0.87 * large, f"{small / large:.2f}"
+    tied, spread = time(np.ones(262144, np.float32), 64), time(_logits(262144, 3), 64)
+    assert tied < 1.32 * spread, f"{tied / spread:.2f}"
 
 
 def test_first_candidate_is_the_fused_argmax(gpu):
