@@ -10,15 +10,18 @@
 //    F = MAGIC + 16 sumi (|16 sumi| <= 2^19, exact), and
 //    fma(F, d_w / 16, -MAGIC * d_w / 16) is sumi * d_w rounded once: F and
 //    the 13-bit product MAGIC * d_w / 16 are exact for every finite scale. An
-//    infinite or NaN d_w gives NaN here, whatever the contract gives, and a
-//    NaN stays: a workgroup with an output that comes out NaN looks its rows'
-//    scales over, and if one is not finite runs its tile once more by the
-//    contract's own four operations: 2048 x 8192 at 512 tokens 40 us, 44 with
-//    every output NaN from the activations, 79 with a bad scale in every row
-//    (each NaN output by itself in one lane had taken 1,855). (With finite d_w the first product is the
-//    contract's, so a NaN from d_x is too. Only a zero's sign may differ: an
-//    accumulator starts at +0.0f and never sees it, and a NaN made of it and
-//    an infinite d_x has the same bits either way.)
+//    infinite or NaN d_w gives NaN here, whatever the contract gives, in every
+//    token of the row. So each wave looks at one token's accumulators before
+//    the tree, and a workgroup with a NaN among them looks its rows' scales
+//    over, and if one is not finite runs its tile once more by the contract's
+//    own four operations: 2048 x 8192 at 512 tokens 40 us, 44 with every
+//    output NaN from the activations, 79 with a bad scale in every row (each
+//    NaN output by itself in one lane had taken 1,855). (A vote on the outputs
+//    was 0.2 us a launch slower: a barrier of its own.)
+//    With finite d_w the first product is the contract's, and so are NaNs from
+//    d_x. Only a zero's sign may differ: an accumulator starts at +0.0f and
+//    never sees it, and a NaN made of it and an infinite d_x has the same bits
+//    either way.
 //  * A wave's tile is 64 rows x 64 tokens (64 x 32 where that leaves CUs
 //    idle), so that a block's weights are unpacked once for 64 tokens and
 //    each operand read from LDS meets four MFMAs.
@@ -103,7 +106,7 @@ struct TileGeo {
     static constexpr int D_LOADS = TT / 32;
     static constexpr int LOADS = 1 + X_LOADS;    // of every wave; one more in the first 1 + D_LOADS
     static_assert(X_OFF == 1024 * (WAVES + 1) && TT % (4 * WAVES) == 0, "the loads below");
-    static_assert(2 * (LDS + 1024) <= 160 * 1024, "two workgroups a CU, the vote's words among them");
+    static_assert(2 * (LDS + 1024) <= 160 * 1024, "two workgroups a CU, the flag and the vote's words among them");
 };
 
 template <int NT>
@@ -249,7 +252,7 @@ struct TileKernel {
 
     // Exchange of token tiles 2 h and 2 h + 1: the tree over the eight
     // accumulators, and the stores.
-    static __device__ __forceinline__ bool reduce_half(const TileParams &P, int n0, int m0, uint8_t *ex, int w, int lane, int h,
+    static __device__ __forceinline__ void reduce_half(const TileParams &P, int n0, int m0, uint8_t *ex, int w, int lane, int h,
                                                        const float acc[NT][RT][4]) {
         const int j = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -269,23 +272,18 @@ struct TileKernel {
                             ((l[0].y + l[1].y) + (l[2].y + l[3].y)) + ((l[4].y + l[5].y) + (l[6].y + l[7].y)),
                             ((l[0].z + l[1].z) + (l[2].z + l[3].z)) + ((l[4].z + l[5].z) + (l[6].z + l[7].z)),
                             ((l[0].w + l[1].w) + (l[2].w + l[3].w)) + ((l[4].w + l[5].w) + (l[6].w + l[7].w))};
-        bool nan = false;
         if (row < P.rows) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (tok + e < P.m) {
-                    P.y[(size_t)(tok + e) * P.rows + row] = v[e];
-                    nan = nan || v[e] != v[e];
-                }
+                if (tok + e < P.m) P.y[(size_t)(tok + e) * P.rows + row] = v[e];
         }
-        return nan;
     }
 
     // The item at rows n0 .., tokens m0 ..: chunk c is computed from LDS
-    // buffer c % 2 while the loads of chunk c + 1 fill the other. Whether an
-    // output of this thread came out NaN.
+    // buffer c % 2 while the loads of chunk c + 1 fill the other. Sets *nan
+    // (0 before) if a row's first token is NaN in a wave's accumulator.
     template <bool PLAIN>
-    static __device__ __forceinline__ bool pass(const TileParams &P, int n0, int m0, uint8_t *lds) {
+    static __device__ __forceinline__ void pass(const TileParams &P, int n0, int m0, uint8_t *lds, int *nan) {
         const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
         int lane = threadIdx.x & 63;
         if constexpr (PLAIN) __asm__ volatile("" : "+v"(lane));   // else the first pass's offsets are kept for this one, and spill
@@ -319,13 +317,17 @@ struct TileKernel {
             arrive();
             if (c + 2 >= chunks) break;
         }
-        bool nan = false;
+        if constexpr (!PLAIN) {
+            bool any = false;
+#pragma unroll
+            for (int r = 0; r < RT; ++r) any = any || acc[0][r][0] != acc[0][r][0];
+            if (any) *nan = 1;
+        }
 #pragma unroll
         for (int h = 0; h < NT / 2; ++h) {
             if (h) __syncthreads();                              // the half before is read
-            nan = reduce_half(P, n0, m0, lds, w, lane, h, acc) || nan;
+            reduce_half(P, n0, m0, lds, w, lane, h, acc);
         }
-        return nan;
     }
 
     // Whether one of the blocks this thread looks at (a row's b, b + 8, ..) has a scale that is not finite.
@@ -340,10 +342,12 @@ struct TileKernel {
         return bad;
     }
 
-    static __device__ __forceinline__ void run(const TileParams &P, int n0, int m0, uint8_t *lds) {
-        // (the votes' barriers keep the exchange until every wave has read it)
-        if (!__syncthreads_or(pass<false>(P, n0, m0, lds))) return;
-        if (__syncthreads_or(scale_not_finite(P, n0))) pass<true>(P, n0, m0, lds);
+    static __device__ __forceinline__ void run(const TileParams &P, int n0, int m0, uint8_t *lds, int *nan) {
+        if (threadIdx.x == 0) *nan = 0;                          // before the barriers of the chunks
+        pass<false>(P, n0, m0, lds, nan);
+        if (*nan == 0) return;                                   // set before the exchange's barrier
+        // (the vote's barriers keep the exchange until every wave has read it)
+        if (__syncthreads_or(scale_not_finite(P, n0))) pass<true>(P, n0, m0, lds, nan);
     }
 };
 static_assert(THREADS == 8 * TILE_ROWS, "scale_not_finite: eight threads a row");
@@ -351,6 +355,7 @@ static_assert(THREADS == 8 * TILE_ROWS, "scale_not_finite: eight threads a row")
 template <int NT>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_tiles_kernel(TileParams P) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ int nan;
     // Workgroups go to the XCDs in turn: each XCD takes a contiguous run of
     // items, token groups fastest, so its L2 serves a row group's weights to
     // all token groups and the activations to all its row groups.
@@ -361,9 +366,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))
     const int n0 = rg * TILE_ROWS, m0 = (item - rg * tgs) * 16 * NT;
     // A last group of at most 32 tokens works on 32.
     if (NT == 4 && P.m - m0 <= 32)
-        TileKernel<2>::run(P, n0, m0, lds);
+        TileKernel<2>::run(P, n0, m0, lds, &nan);
     else
-        TileKernel<NT>::run(P, n0, m0, lds);
+        TileKernel<NT>::run(P, n0, m0, lds, &nan);
 }
 
 template <int NT>
