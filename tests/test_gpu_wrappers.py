@@ -95,3 +95,25 @@ def test_good_out_still_works(gpu, t):
     torch.cuda.synchronize()
     assert got.data_ptr() == y.data_ptr()
     assert bool(torch.all(y[:ROWS] == 0)) and bool(torch.all(torch.isnan(y[ROWS:])))
+
+
+@pytest.mark.parametrize("raw", [True, False])
+def test_calls_run_on_the_current_stream(gpu, t, monkeypatch, raw):
+    """The handle the calls pass is the device's current stream's, on the default stream, a
+    side stream and a capturing one, with and without torch's raw-handle function."""
+    import torch
+    if not raw:
+        monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    monkeypatch.setattr(gpu, "_raw_stream", None)
+    x = t["x"]
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    assert gpu._stream(x) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert gpu._stream(x) == side.cuda_stream
+    with torch.cuda.graph(graph, stream=side):
+        assert gpu._stream(x) == side.cuda_stream
+        y = gpu.gemv_q4_0_f32(t["blocks"], K, x)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert not y.any()                       # zero weights
