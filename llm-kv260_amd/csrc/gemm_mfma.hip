@@ -115,7 +115,7 @@ struct Geo {
     // fp32 scales [8 D blocks][XDP], tokens along a row. The pitch makes the
     // transposing writes (64 / TT pieces of consecutive tokens per wave
     // instruction, four rows apart) fall in distinct banks.
-    static constexpr int XDP = TT < 64 ? TT + TT / 4 : TT;
+    static constexpr int XDP = TT + TT / 4;
     static constexpr int XD_OFF = X_OFF + TT * AP;
     static constexpr int BUF = XD_OFF + 8 * D * XDP * 4;    // one round
     // Exchange of the eight accumulators: [8][TT][EXP] fp32. Two of them

@@ -142,7 +142,7 @@ struct TileKernel {
     // Where an item's chunks are loaded from. A row past the last or a token
     // past m lies beyond the resources' sizes and is not read (a lane's
     // offset says which row or token; the chunk's comes with the
-    // instruction); past the last item the sizes are zero.
+    // instruction).
     struct Source {
         v4i w, x, p;
         int w_at, x_at, p_at, p_step;
