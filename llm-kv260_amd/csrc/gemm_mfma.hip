@@ -453,7 +453,7 @@ void gemm_mfma_kernel(GemmParams Pm) {
 constexpr int DEPTH = 2;
 
 template <int MT, int D, int OCC, int NRL = 16>
-hipError_t launch_geo(const GemmParams &Pm, hipStream_t stream) {
+hipError_t launch_geo(const GemmParams &Pm, int cus, hipStream_t stream) {
     using G = Geo<MT, D, DEPTH, OCC, NRL>;
     const void *fn = reinterpret_cast<const void *>(&gemm_mfma_kernel<MT, D, DEPTH, OCC, NRL>);
     hipError_t e = allow_dynamic_lds(fn, LDS_MAX);
@@ -463,7 +463,7 @@ hipError_t launch_geo(const GemmParams &Pm, hipStream_t stream) {
     if (e != hipSuccess) return e;
     if (per_cu < 1) per_cu = 1;
     const long items = (long)((Pm.rows + NRL - 1) / NRL) * ((Pm.m + G::TT - 1) / G::TT);
-    long grid = (long)device_cu_count() * per_cu;
+    long grid = (long)cus * per_cu;
     if (grid > items) grid = items;
     hipLaunchKernelGGL((gemm_mfma_kernel<MT, D, DEPTH, OCC, NRL>), dim3((unsigned)grid), dim3(GTHREADS), G::LDS, stream,
                        Pm);
@@ -473,34 +473,33 @@ hipError_t launch_geo(const GemmParams &Pm, hipStream_t stream) {
 // Chunks per round: the largest power of two up to DMAX that divides the
 // K / 256 chunks of a row, so that every item is whole rounds.
 template <int MT, int DMAX, int OCC, int NRL = 16>
-hipError_t launch_mt(const GemmParams &Pm, hipStream_t stream) {
+hipError_t launch_mt(const GemmParams &Pm, int cus, hipStream_t stream) {
     const int C = Pm.k / 256;
     if constexpr (DMAX >= 8) {
-        if (C % 8 == 0) return launch_geo<MT, 8, OCC, NRL>(Pm, stream);
+        if (C % 8 == 0) return launch_geo<MT, 8, OCC, NRL>(Pm, cus, stream);
     }
     if constexpr (DMAX >= 4) {
-        if (C % 4 == 0) return launch_geo<MT, 4, OCC, NRL>(Pm, stream);
+        if (C % 4 == 0) return launch_geo<MT, 4, OCC, NRL>(Pm, cus, stream);
     }
     if constexpr (DMAX >= 2) {
-        if (C % 2 == 0) return launch_geo<MT, 2, OCC, NRL>(Pm, stream);
+        if (C % 2 == 0) return launch_geo<MT, 2, OCC, NRL>(Pm, cus, stream);
     }
-    return launch_geo<MT, 1, OCC, NRL>(Pm, stream);
+    return launch_geo<MT, 1, OCC, NRL>(Pm, cus, stream);
 }
 
 // Workgroups per CU.
 constexpr int GEMM_OCC = 2;
 
-hipError_t launch_tokens(const GemmParams &Pm, hipStream_t stream) {
+hipError_t launch_tokens(const GemmParams &Pm, int cus, hipStream_t stream) {
     // 16 or 32 tokens per item. With several token groups the weights are read
     // once per group, the later reads mostly from the caches. A round holds
     // 128 (or, at two workgroups per CU, 64) token-chunks of activations.
     constexpr int OCC = GEMM_OCC;
-    const int cus = device_cu_count();
     const int mt = gemm_route::split_tokens(Pm.m, Pm.rows, Pm.k, cus) / 16;
     if (gemm_route::split_rows(Pm.m, Pm.rows, Pm.k, cus) == 8)
-        return launch_mt<1, 8, 1, 8>(Pm, stream);
-    if (mt == 1) return launch_mt<1, 8 / OCC, OCC>(Pm, stream);
-    return launch_mt<2, 4 / OCC, OCC>(Pm, stream);
+        return launch_mt<1, 8, 1, 8>(Pm, cus, stream);
+    if (mt == 1) return launch_mt<1, 8 / OCC, OCC>(Pm, cus, stream);
+    return launch_mt<2, 4 / OCC, OCC>(Pm, cus, stream);
 }
 
 }  // namespace
@@ -528,10 +527,11 @@ hipError_t launch_gemm(const MatrixRef &w, const uint8_t *x, int m, float *y, hi
     if ((size_t)P.rows * (size_t)(P.k / QK * Q4_0_BYTES) >= 0x7fff0000u ||
         (size_t)64 * P.rows * 4 >= 0x7fff0000u)
         return hipErrorInvalidValue;
-    switch (gemm_route::form(m, P.rows, P.k, device_cu_count())) {
+    const int cus = device_cu_count();   // (asks HIP for the device: once a call)
+    switch (gemm_route::form(m, P.rows, P.k, cus)) {
         case gemm_route::ROWS: return launch_gemm_rows(P.w, x, m, y, P.rows, P.k, stream);
-        case gemm_route::TILES: return launch_gemm_tiles(P.w, x, m, y, P.rows, P.k, stream);
-        default: return launch_tokens(P, stream);   // at most two covers of 32-token items: the outputs fit a range too
+        case gemm_route::TILES: return launch_gemm_tiles(P.w, x, m, y, P.rows, P.k, cus, stream);
+        default: return launch_tokens(P, cus, stream);   // at most two covers of 32-token items: the outputs fit a range too
     }
 }
 

@@ -387,7 +387,8 @@ hipError_t launch_tiles(TileParams P, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_gemm_tiles(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, hipStream_t stream) {
+hipError_t launch_gemm_tiles(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, int cus,
+                             hipStream_t stream) {
     TileParams P{};
     P.w = w;
     P.x = x;
@@ -400,7 +401,7 @@ hipError_t launch_gemm_tiles(const uint8_t *w, const uint8_t *x, int m, float *y
     // is its chunks' (2048 x 8192 at 256 tokens: 26 us against 37). Past that
     // 64-token tiles, 4% slower to 25% faster (gate|up 8% at 512 tokens).
     const long row_groups = (rows + TILE_ROWS - 1) / TILE_ROWS;
-    if (row_groups * ((m + 31) / 32) <= device_cu_count()) return launch_tiles<2>(P, stream);
+    if (row_groups * ((m + 31) / 32) <= cus) return launch_tiles<2>(P, stream);
     return launch_tiles<4>(P, stream);
 }
 

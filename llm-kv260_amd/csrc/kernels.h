@@ -88,7 +88,8 @@ hipError_t launch_gemv_mt(const uint8_t *w, const uint8_t *x, int m, float *y, i
 bool gemm_rows_fits(int rows, int k);
 hipError_t launch_gemm_rows(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, hipStream_t stream);
 // Many tokens in one launch (gemm_tiles.hip): any m, rows and k whose weights fit a 32-bit byte count.
-hipError_t launch_gemm_tiles(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, hipStream_t stream);
+hipError_t launch_gemm_tiles(const uint8_t *w, const uint8_t *x, int m, float *y, int rows, int k, int cus,
+                             hipStream_t stream);
 
 // x: float32[m][K] -> engine layout rows, or ggml Q8_0 block rows.
 hipError_t launch_quantize_q8_0(const float *x, int k, int m, uint8_t *out, XFormat out_fmt, hipStream_t stream);
