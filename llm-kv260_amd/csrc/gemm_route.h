@@ -39,7 +39,7 @@ inline int split_tokens(int m, int rows, int k, int cus) {
 // long rows (k >= 8192: down), while 8-row items cover the CUs once: eight
 // chunks a round, one workgroup a CU, 2048 x 8192 at 5 to 16 tokens in 9.2-10.1
 // us against 10.4-10.6. Past that a CU runs two of them one after the other
-// (3072 x 8192 at 16 16.3 against 10.6, 3072 x 16128 72 against 37), and at k =
+// (3072 x 8192 at 16 16.2 against 10.5, 3072 x 16128 72 against 37), and at k =
 // 2048 (o, q|k|v) they were slower too.
 inline int split_rows(int m, int rows, int k, int cus) {
     return m <= 16 && k >= 8192 && (rows + 7) / 8 <= cus ? 8 : 16;
@@ -75,11 +75,11 @@ inline bool tiles_faster(int m, int rows, int k, int cus) {
 enum Form { SPLIT, ROWS, TILES };   // gemm_mfma.hip, gemm_rows.hip, gemm_tiles.hip
 
 // From ROWS_MIN rows on (and k a multiple of its 512-value segments) the
-// row-split kernel takes up to 16 tokens: at 8192 x 2048 6.6 us at 16 tokens
-// against 8.3 in the whole-prompt kernel, which has 8.3 against 9.3 at 17;
-// gate|up 7.9 and 9.0 at 16, 10.2 and 9.5 at 24; the LM head 47 and 59 at 16,
-// 80 and 51 at 17. (At 3,072 rows it was twice as slow as the class-split
-// kernel: 48 workgroups.) Up to 32 tokens it stays ahead on longer rows while
+// row-split kernel takes up to 16 tokens: 8200 x 2048 7.1 us at 16 tokens
+// against 9.3 in the whole-prompt kernel, which has 9.4 against 9.6 at 17;
+// gate|up 8.1 and 9.9 at 16, 10.3 and 10.1 at 24; 32000 x 2048 13.6 and 14.4
+// at 16, 18.6 and 14.4 at 17. (At 3,072 rows it was twice as slow as the
+// class-split kernel: 48 workgroups.) Up to 32 tokens it stays ahead on longer rows while
 // its workgroups of 64 rows are one cover of the CUs: 16384 x 8192 at 32
 // tokens 28.5 against 31.6, 8192 x 16384 50.4 against 55.9; at k = 2048 even,
 // and past one cover it loses (28672 x 8192 53.8 against 41.8).

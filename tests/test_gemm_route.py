@@ -80,8 +80,8 @@ ROW_TIMES = (
 
 # m, rows, k, then microseconds: row-split and whole-prompt kernel, matrices of many rows.
 MANY_ROWS_TIMES = (
-    (16, 8192, 2048, 6.6, 8.3), (17, 8192, 2048, 9.3, 8.3), (24, 16384, 2048, 10.2, 9.5), (16, 128256, 2048, 47, 59),
-    (17, 128256, 2048, 80, 51), (32, 8192, 8192, 27.2, 29.1), (32, 9216, 4096, 15.7, 16.6), (28, 12288, 8192, 27.8, 29.4),
+    (16, 8200, 2048, 7.1, 9.3), (17, 8200, 2048, 9.6, 9.4), (24, 16384, 2048, 10.3, 10.1), (16, 32000, 2048, 13.6, 14.4),
+    (17, 32000, 2048, 18.6, 14.4), (17, 128256, 2048, 73.4, 51.5), (32, 8192, 8192, 27.2, 29.1), (32, 9216, 4096, 15.7, 16.6), (28, 12288, 8192, 27.8, 29.4),
     (17, 16384, 8192, 28.5, 30.5), (32, 16384, 4096, 16.6, 17.5), (32, 16384, 16384, 52.4, 59.0),
     (32, 28672, 8192, 53.8, 41.8), (17, 28672, 4096, 30.3, 24.7), (33, 16384, 8192, 41.8, 39.3),
 )
