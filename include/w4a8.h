@@ -130,7 +130,7 @@ int w4a8_topk_no_alloc(const float *y, int n, int k, float *vals, int32_t *idx, 
  *     through ggml's vector expf; the input of down (:858-860). y = W Q8_0(a).
  * Each is byte-identical to the standalone producer below followed by
  * w4a8_gemv. x, norm_w and gate_up 16-byte aligned; the fused rmsnorm takes
- * k <= 8192, the standalone one any k.
+ * k <= 8192, the standalone one k <= 16384.
  * The float64 sum is taken in parallel with a bound on the reference order's
  * result, and in that order itself only where the bound does not settle the
  * float32 it rounds to.

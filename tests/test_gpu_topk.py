@@ -116,9 +116,9 @@ def test_topk_time_where_the_bound_does_not_help(gpu):
             best = min(best, start.elapsed_time(end))
         return best
 
-    small, large = time(_logits(1000, 1), 1), time(_logits(128256, 2), 40)
+    large, small = time(_logits(128256, 2), 40), time(_logits(1000, 1), 1)
     assert small < 0.87 * large, f"{small / large:.2f}"
-    tied, spread = time(np.ones(262144, np.float32), 64), time(_logits(262144, 3), 64)
+    spread, tied = time(_logits(262144, 3), 64), time(np.ones(262144, np.float32), 64)
     assert tied < 1.32 * spread, f"{tied / spread:.2f}"
 
 
